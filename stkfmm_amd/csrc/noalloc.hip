@@ -17,6 +17,7 @@
 #include <mutex>
 
 #include "../../include/stkfmm_p2p.h"
+#include "p2p_direct_layout.hpp"
 #include "p2p_internal.hpp"
 
 namespace stkp2p {
@@ -27,25 +28,28 @@ constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// device address of `scratch` on each device (the host-side name is not a device address)
-void *g_scratch_ptr[kMaxDevices] = {};
+// partial sums of the chunked direct sums of the other entries, which may run beside a no-alloc call
+static __device__ __align__(256) double direct_partial[16 * kDirectPartialTargets];
+
+// device addresses of the two arrays on each device (the host-side names are not device addresses)
+void *g_scratch_ptr[kMaxDevices] = {}, *g_partial_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
 
-int scratch_ptr(int dev, unsigned char **out) {
+int symbol_ptr(int dev, void **cache, const void *symbol, const char *name, void **out) {
     if (dev < 0 || dev >= kMaxDevices)
-        return report_error(STKFMM_ERR_UNSUPPORTED, "no-alloc direct sum: device index out of range");
+        return report_error(STKFMM_ERR_UNSUPPORTED, "direct sum: device index out of range");
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_ptr[dev]) {
+    if (!cache[dev]) {
         void *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        const hipError_t e = hipGetSymbolAddress(&p, symbol);
         if (e != hipSuccess || !p) {
             char buf[256];
-            snprintf(buf, sizeof(buf), "no-alloc direct sum: hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
+            snprintf(buf, sizeof(buf), "direct sum: hipGetSymbolAddress(%s): %s", name, hipGetErrorString(e));
             return report_error(STKFMM_ERR_HIP, buf);
         }
-        g_scratch_ptr[dev] = p;
+        cache[dev] = p;
     }
-    *out = (unsigned char *)g_scratch_ptr[dev];
+    *out = cache[dev];
     return STKFMM_OK;
 }
 
@@ -130,6 +134,16 @@ int fail(int code, const char *fmt, long long a = 0, long long b = 0) {
 }
 
 } // namespace
+
+int direct_partial_ptr(double **out) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess)
+        return report_error(STKFMM_ERR_HIP, "direct sum: hipGetDevice failed");
+    void *p = nullptr;
+    const int rc = symbol_ptr(dev, g_partial_ptr, HIP_SYMBOL(direct_partial), "direct_partial", &p);
+    *out = (double *)p;
+    return rc;
+}
 } // namespace stkp2p
 
 using namespace stkp2p;
@@ -155,14 +169,15 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess)
         e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-    const int T = direct_targets_per_lane(nTrg), TT = kWave * T;
+    const int T = nTrg < 32768 ? 1 : 2, TT = kWave * T; // the work list's targets per lane
     if (e == hipSuccess)
         e = items_occupancy(uk, precision, T, &bpc);
     if (e != hipSuccess)
         return fail(STKFMM_ERR_HIP, "no-alloc direct sum: device query failed");
-    unsigned char *base = nullptr;
-    if ((rc = scratch_ptr(dev, &base)))
+    void *scratch_mem = nullptr;
+    if ((rc = symbol_ptr(dev, g_scratch_ptr, HIP_SYMBOL(scratch), "scratch", &scratch_mem)))
         return rc;
+    unsigned char *const base = (unsigned char *)scratch_mem;
     bpc = bpc < 1 ? 1 : bpc;
 
     const int ks = uker_ks(uk), ks1 = uker_ks1(uk), kt = uker_kt(uk);
@@ -170,7 +185,8 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
     // the plan's chunking, or fewer and longer chunks when its partial sums do not fit
     long long max_src = default_max_src((long long)nSrc * n_tiles, (long long)n_cu * bpc);
     long long nc = (nSrc + max_src - 1) / max_src;
-    if (layout(n_tiles * nc, n_tiles, kt, TT).end > kScratchBytes) {
+    const bool limited = layout(n_tiles * nc, n_tiles, kt, TT).end > kScratchBytes;
+    if (limited) {
         const Layout one = layout(n_tiles, n_tiles, kt, TT);
         if (one.end > kScratchBytes)
             return fail(STKFMM_ERR_ARG,
@@ -185,6 +201,27 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
             --nc_max;
         max_src = (nSrc + nc_max - 1) / nc_max;
         nc = (nSrc + max_src - 1) / max_src;
+    }
+    // One launch (p2p_direct.hpp), whose partial sums always fit the array.  The work list below remains
+    // for the mixed-mode sums that do not run so (direct_in_one_launch), and for those above the array's
+    // size: their longer chunks need not start on a whole source tile, which decides the sources each
+    // FP32 partial sum holds.
+    if ((precision == STKFMM_PREC_FP64 || (!limited && direct_in_one_launch(precision, uk))) && nSrc <= (1 << 30) && nTrg <= (1 << 30)) {
+        DirectArgs a{};
+        a.sc = DArr{d_srcCoord, 3, 1};
+        a.v1 = DArr{d_srcValue, ks, 1};
+        a.v2 = DArr{d_srcValue + ks1, ks, 1};
+        a.tc = DArr{d_trgCoord, 3, 1};
+        a.out = OArr{d_trgValue, kt, 1};
+        a.partial = (double *)base;
+        a.scale = uker_scale(uk);
+        a.n_src = nSrc;
+        a.n_trg = nTrg;
+        const DirectLayout l = direct_layout(precision, direct_targets_per_lane(precision, kt, nTrg), kt, uker_run(uk), nSrc,
+                                             nTrg, n_cu);
+        if ((e = launch_direct(uk, precision, a, l, s)) != hipSuccess)
+            return fail(STKFMM_ERR_HIP, "no-alloc direct sum: launch failed");
+        return STKFMM_OK;
     }
     const long long n_items = n_tiles * nc;
     if (n_items > (1LL << 30))

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/stkfmm_p2p.h"
+#include "p2p_direct_layout.hpp"
 #include "p2p_internal.hpp"
 
 using namespace stkp2p;
@@ -271,6 +272,10 @@ struct stkfmm_plan {
     // launch variant of the LDS item kernel: precision, or kPrecMixedFar (mixed with the far-tile
     // displacement) for tree-derived mixed work lists at T = 2
     int kernel_prec = 0;
+    // one group, one range, default tuning: the whole plan is one direct-sum launch (p2p_direct.hpp)
+    bool direct = false;
+    DirectLayout dlayout{};
+    int dt_begin = 0, ds_begin = 0, dn_trg = 0, dn_src = 0; // its target and source range
     int level_min = 0, n_copies = 0, rec_words = 0;
     double *d_recs = nullptr;
     // sort_points: Morton ordering of each execute's points (morton.hip) into the SoA copies below
@@ -351,6 +356,13 @@ static void group_tiles(int n, int TT, bool pieces, std::vector<int> &counts) {
         counts.push_back(q);
         n -= q;
     }
+}
+
+// sizes a direct sum's 32-bit indices cover
+static bool direct_sizes(int n_src, int n_trg) { return n_src <= (1 << 30) && n_trg <= (1 << 30); }
+// direct sums whose entry orders the points (or whose sizes one launch does not cover)
+static bool direct_sorts_points(int n_src, int n_trg) {
+    return (n_src >= kDirectSortMin && n_trg >= kDirectSortMin) || !direct_sizes(n_src, n_trg);
 }
 
 extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision, int n_src, int n_trg,
@@ -652,6 +664,33 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     p->pairs = pairs;
     (void)hipGetDevice(&p->device);
 
+    // A single untuned direct sum below the sizes that pay for ordered points: one launch instead of queue
+    // reset, item kernel and reduce (above, the item kernel is the faster one: 65,536^2 PVel FP64 as given
+    // 4.0 against 4.3 ms).  The item list above stays for stkfmm_plan_stats.
+    const stkfmm_tune no_tune{};
+    if (n_groups == 1 && !grp_level && std::memcmp(&tn, &no_tune, sizeof(tn)) == 0 && p->n_items > 0 &&
+        grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && !direct_sorts_points(n_src, n_trg) &&
+        direct_in_one_launch(precision, uk)) {
+        const int r0 = grp_rng_ptr[0];
+        p->direct = true;
+        p->dt_begin = grp_trg_begin[0];
+        p->dn_trg = grp_trg_end[0] - p->dt_begin;
+        p->ds_begin = rng_src_begin[r0];
+        p->dn_src = rng_src_end[r0] - p->ds_begin;
+        p->dlayout = direct_layout(precision, precision == STKFMM_PREC_FP64 ? direct_fp64_targets(p->KT) : T, p->KT, uker_run(uk), p->dn_src,
+                                   p->dn_trg, n_cu);
+        if (p->dlayout.chunks > 1) {
+            const hipError_t e = hipMalloc((void **)&p->d_partial,
+                                           sizeof(double) * p->dlayout.chunks * p->KT * (size_t)p->dn_trg);
+            if (e != hipSuccess) {
+                plan_free(p);
+                return hip_error(e, "plan workspace");
+            }
+        }
+        *plan_out = p;
+        return STKFMM_OK;
+    }
+
     int r;
     if ((r = upload(&p->d_items, items, "plan items")) || (r = upload(&p->d_ranges, ranges, "plan ranges")) ||
         (r = upload(&p->d_tiles, tiles, "plan tiles")) || (r = upload(&p->d_qptr, q_ptr, "plan queues"))) {
@@ -708,6 +747,25 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
 
 static bool arr_ok(const stkfmm_array *a) { return a && a->ptr && a->stride >= 0 && a->fstride >= 0; }
 
+// one direct-sum launch over arrays that start at the first source and target
+static int enqueue_direct(int uk, int prec, const DirectLayout &l, int n_src, int n_trg, const DArr &sc, const DArr &v1,
+                          const DArr &v2, const DArr &tc, const OArr &out, const int *perm, double *partial,
+                          hipStream_t s) {
+    DirectArgs a{};
+    a.sc = sc;
+    a.v1 = v1;
+    a.v2 = v2;
+    a.tc = tc;
+    a.out = out;
+    a.perm = perm;
+    a.partial = partial;
+    a.scale = uker_scale(uk);
+    a.n_src = n_src;
+    a.n_trg = n_trg;
+    HIP_TRY(launch_direct(uk, prec, a, l, s), "direct sum launch");
+    return STKFMM_OK;
+}
+
 static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_array *sv, const stkfmm_array *sv2,
                         const stkfmm_array *tc, const stkfmm_out_array *tv, const int *perm, hipStream_t s,
                         bool allow_timing) {
@@ -722,6 +780,26 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
     a.v1 = DArr{sv->ptr, sv->stride, sv->fstride};
     a.v2 = (p->KS1 < p->KS) ? DArr{sv2->ptr, sv2->stride, sv2->fstride} : a.v1;
     a.tc = DArr{tc->ptr, tc->stride, tc->fstride};
+    if (p->direct) {
+        const long long s0 = p->ds_begin, t0 = p->dt_begin;
+        auto from = [](const DArr &x, long long i) { return DArr{x.p + i * x.s, x.s, x.fs}; };
+        const OArr out{tv->ptr + (perm ? 0 : t0 * tv->stride), tv->stride, tv->fstride};
+        const bool timed = allow_timing && p->timing;
+        hipEvent_t *ev = timed ? &p->ev[3 * (p->n_timed % stkfmm_plan::kRing)] : nullptr;
+        if (timed) {
+            ++p->n_timed;
+            HIP_TRY(hipEventRecord(ev[0], s), "event record");
+        }
+        const int rc = enqueue_direct(p->uk, p->prec, p->dlayout, p->dn_src, p->dn_trg, from(a.sc, s0), from(a.v1, s0),
+                                      from(a.v2, s0), from(a.tc, t0), out, perm ? perm + t0 : nullptr, p->d_partial, s);
+        if (rc)
+            return rc;
+        if (timed) { // the partial sums of a chunked sum are added inside the first interval
+            HIP_TRY(hipEventRecord(ev[1], s), "event record");
+            HIP_TRY(hipEventRecord(ev[2], s), "event record");
+        }
+        return STKFMM_OK;
+    }
     if (p->sorted) {
         // order the points of this execute, then run on the sorted SoA copies
         SortArgs so;
@@ -931,7 +1009,7 @@ extern "C" int stkfmm_plan_destroy(stkfmm_plan *p) {
 namespace {
 std::mutex g_mu;
 
-// cache of single-group plans for direct sums, keyed by shape
+// cache of the plans of direct sums that do not run in one launch, keyed by shape
 struct DirectKey {
     int device, uk, prec, n_src, n_trg;
     bool operator==(const DirectKey &o) const {
@@ -953,26 +1031,15 @@ int direct_plan(int uk, int prec, int n_src, int n_trg, stkfmm_plan **out) {
         }
     }
     const int gb = 0, ge = n_trg, gp[2] = {0, 1}, rb = 0, re = n_src;
-    // one target group.  From 16,384 sources and targets on, the points are ordered along a Morton
-    // curve at every call (sort_points, T = 2): measured on MI355X, whole call including the ordering,
-    // 65,536^2 PVel 3.94 -> 3.77 ms FP64 (LDS staging; 3.76 with scalar broadcast on a box where the
-    // unordered call took 4.03) and 2.88 -> 2.70 ms mixed, 131,072^2 Stokeslet mixed 9.97 -> 8.43 ms,
-    // 16,384^2 about even, 8192^2 slower (0.11 -> 0.14 ms: the ordering's fixed cost).
-    // Below that: one target per lane under 32,768 targets (twice the waves for a small sum), and in
-    // FP64 the scalar-broadcast staging at or above it (8192^2 LapPGrad 0.127 -> 0.100 ms FP64 and
-    // 0.115 -> 0.096 ms mixed at T = 1).  Only the target-to-lane mapping and the staging change, not
-    // the order in which a target sums its sources.
+    // One target group.  From kDirectSortMin sources and targets its points are ordered along a Morton
+    // curve at every call: T = 2, and in FP64 the scalar-broadcast records (65,536^2 PVel FP64 4.05 ->
+    // 3.76 ms, 131,072^2 14.72 -> 14.24 ms against LDS staging of the ordered points).  Below that, where
+    // one launch does not serve (direct_in_one_launch): one target per lane under 32,768 targets.
     stkfmm_tune tn{};
-    const bool small = direct_targets_per_lane(n_trg) == 1;
-    tn.targets_per_lane = direct_targets_per_lane(n_trg);
-    tn.broadcast = (!small && prec == STKFMM_PREC_FP64) ? 1 : 0;
-    if (n_trg >= kDirectSortMin && n_src >= kDirectSortMin) {
-        // ordered points: T = 2, and in FP64 the scalar-broadcast records (65,536^2 PVel FP64 4.05 ->
-        // 3.76 ms, 131,072^2 14.72 -> 14.24 ms against LDS staging of the ordered points)
-        tn.sort_points = 1;
-        tn.targets_per_lane = 2;
-        tn.broadcast = (prec == STKFMM_PREC_FP64) ? 1 : 0;
-    }
+    const bool sort = n_trg >= kDirectSortMin && n_src >= kDirectSortMin;
+    tn.sort_points = sort ? 1 : 0;
+    tn.targets_per_lane = sort || n_trg >= 32768 ? 2 : 1;
+    tn.broadcast = (sort && prec == STKFMM_PREC_FP64) ? 1 : 0;
     stkfmm_plan *p = nullptr;
     int rc = stkfmm_plan_create(&p, uk, prec, n_src, n_trg, 1, &gb, &ge, nullptr, gp, &rb, &re, &tn);
     if (rc)
@@ -1027,11 +1094,21 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
         return STKFMM_OK;
     if (!sc || !sv || !tc || !tv)
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
-    stkfmm_plan *p = nullptr;
-    int rc = direct_plan(uk, prec, n_src, n_trg, &p);
-    if (rc)
-        return rc;
     const int ks = uker_ks(uk), ks1 = uker_ks1(uk), kt = uker_kt(uk);
+    int rc;
+    if (!direct_sorts_points(n_src, n_trg) && direct_in_one_launch(prec, uk)) {
+        int n_cu = 0;
+        double *partial = nullptr;
+        if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
+            return rc;
+        const DirectLayout l = direct_layout(prec, direct_targets_per_lane(prec, kt, n_trg), kt, uker_run(uk), n_src, n_trg,
+                                             n_cu);
+        return enqueue_direct(uk, prec, l, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
+                              DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, partial, s);
+    }
+    stkfmm_plan *p = nullptr;
+    if ((rc = direct_plan(uk, prec, n_src, n_trg, &p)))
+        return rc;
     stkfmm_array a_sc{sc, 3, 1}, a_sv{sv, ks, 1}, a_sv2{sv + ks1, ks, 1}, a_tc{tc, 3, 1};
     stkfmm_out_array a_tv{tv, kt, 1};
     return plan_enqueue(p, &a_sc, &a_sv, &a_sv2, &a_tc, &a_tv, nullptr, s, false);

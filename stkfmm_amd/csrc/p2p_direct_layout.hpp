@@ -1,0 +1,78 @@
+// p2p_direct_layout.hpp -- how a direct sum is cut into workgroups (host side of p2p_direct.hpp).
+#pragma once
+
+#include "p2p_internal.hpp"
+
+namespace stkp2p {
+
+constexpr int kDirectWaves = 8; // waves per workgroup, at most
+
+struct DirectLayout {
+    int T;           // targets per lane
+    int ls;          // log2 lanes per target
+    int unit;        // targets per workgroup, 64*T >> ls
+    int units;       // workgroups over the targets (blockIdx.x)
+    int tail_begin;  // mixed: first target of the partly filled tile whose lanes split the runs, ...
+    int tail_ls;     // ... and its log2 lanes per target (0: no such tile; it is then the last unit)
+    int chunks;      // source chunks (blockIdx.y)
+    int chunk_tiles; // 64-source tiles per chunk
+    int waves;       // waves per workgroup
+};
+
+// The cheapest cut by a model of one CU, in cycles: a wave of a workgroup stages a source tile (kStage)
+// and evaluates its 64 sources with 64*T >> ls pairs each, 64 lanes at a time (about 50 + 15 KT cycles
+// a pair and lane in FP64, 50 + 8 KT in mixed mode); a CU holds ceil(workgroups / CUs) workgroups on
+// four SIMDs, and fewer than about three waves on a SIMD run at the latency of their dependency chain
+// (kAlone).  The partial sums of c chunks cost a second launch and their reads, kReduce + c kChunk.  Fitted
+// to a sweep of ls, chunks and waves over 11 shapes in each precision; the cut taken is within 15 % of
+// the sweep's best (for instance 8192^2 LapPGrad FP64 54 us, best 53; 9,000 x 1,000 PVel 19 us, best 18).
+inline DirectLayout direct_layout(int prec, int T, int kt, int run, int n_src, int n_trg, int n_cu) {
+    const int TT = kWave * T;
+    const long long stiles = (n_src + kSrcTile - 1) / kSrcTile;
+    DirectLayout best{};
+    double best_t = -1.0;
+    const int ls_max = (prec == 0) ? 4 : (run >= 64 ? 0 : (run == 32 ? 1 : 2));
+    const double pair = (prec == 0 ? 50.0 + 15.0 * kt : 50.0 + 8.0 * kt);
+    const double kStage = 800.0, kSetup = 4000.0, kReduce = 8000.0, kChunk = 250.0, kAlone = 3.0;
+    // workgroups of a CU whose set-up (targets, the waves' sums) overlaps others' pairs: by registers
+    const int overlap = kt <= 4 ? 4 : (kt <= 6 ? 1 : 2);
+    const int max_waves = kt > 6 ? kDirectWaves / 2 : kDirectWaves; // 120-156 VGPRs: finer packing
+    for (int ls = 0; ls <= ls_max; ++ls) {
+        DirectLayout l{};
+        l.T = T;
+        l.ls = ls;
+        l.unit = TT >> ls;
+        if (prec != 0) {
+            const int rem = n_trg % TT;
+            l.tail_ls = rem ? tile_lsplit(rem, TT) : 0;
+            l.tail_begin = l.tail_ls ? n_trg - rem : n_trg;
+            l.units = (l.tail_begin + l.unit - 1) / l.unit + (l.tail_ls ? 1 : 0);
+        } else {
+            l.tail_begin = n_trg;
+            l.units = (n_trg + l.unit - 1) / l.unit;
+        }
+        for (int c = 1; c <= stiles; c = (c < 8) ? c + 1 : c + c / 4) {
+            // partial sums of the chunks: at most kDirectPartialTargets targets' worth
+            if (c > 1 && ((long long)c * n_trg > kDirectPartialTargets || c > 65535))
+                break;
+            l.chunk_tiles = (int)((stiles + c - 1) / c);
+            l.chunks = (int)((stiles + l.chunk_tiles - 1) / l.chunk_tiles);
+            l.waves = max_waves;
+            while (l.waves > 1 && l.waves / 2 >= l.chunk_tiles)
+                l.waves /= 2;
+            const double rounds = (double)((l.chunk_tiles + l.waves - 1) / l.waves);
+            const double wave_t = rounds * (kStage + (kWave >> ls) * T * pair);
+            const long long wgs = ((long long)l.units * l.chunks + n_cu - 1) / n_cu;
+            const double per_simd = (double)(wgs * l.waves) / 4.0; // waves a SIMD has to run
+            const double t = kSetup * (double)((wgs + overlap - 1) / overlap) + wave_t * (per_simd > kAlone ? per_simd + 0.25 : kAlone + 0.25) +
+                             (l.chunks > 1 ? kReduce + kChunk * l.chunks : 0.0);
+            if (best_t < 0.0 || t < best_t) {
+                best_t = t;
+                best = l;
+            }
+        }
+    }
+    return best;
+}
+
+} // namespace stkp2p

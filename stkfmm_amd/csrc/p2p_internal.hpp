@@ -89,6 +89,20 @@ struct ReduceArgs {
     double scale;         // ScaleFactor of the kernel
 };
 
+// a direct sum in one launch (p2p_direct.hpp)
+struct DirectArgs {
+    DArr sc, v1, v2, tc; // as ItemArgs
+    OArr out;
+    const int *perm;     // output row of target i (null: identity)
+    double *partial;     // [chunk][KT][n_trg], used when there are several chunks
+    double scale;        // ScaleFactor of the kernel
+    int n_src, n_trg;
+    int ls, unit, tail_begin, tail_ls, chunk_tiles; // DirectLayout
+};
+struct DirectLayout;
+// the chunks' partial sums hold at most this many targets' outputs (16 MiB at 16 outputs)
+constexpr long long kDirectPartialTargets = 131072;
+
 // XCD-contiguous work mapping.  Workgroups of a launch are dealt to MI355X's 8 XCDs round-robin
 // (workgroup b runs on XCD b % 8), each XCD with its own L2.  A launch of 8*ceil(n/8) workgroups that
 // takes unit xcd_unit(b, n) gives XCD x the contiguous units [x*q, (x+1)*q), q = ceil(n/8), so work on
@@ -170,8 +184,10 @@ struct UkerOps {
                               hipStream_t s);
     hipError_t (*occ_sgpr)(int prec, int T, int *blocks);
     hipError_t (*stage)(int prec, const StageArgs &a, int n_copies, hipStream_t s);
+    hipError_t (*direct)(int prec, int T, const DirectArgs &a, const DirectLayout &l, hipStream_t s);
     int words[2]; // scalar-broadcast record size in 8-byte words, FP64 / mixed
     int ks, ks1, kt;
+    int run;      // mixed mode: sources per FP32 partial sum
 };
 
 constexpr int kNumCoreUker = 14;   // micro-kernels 0..13 (p2p_kernels.hip)
@@ -187,9 +203,19 @@ inline long long default_max_src(long long total_cost, long long concurrent) {
     return m > 512 ? m : 512;
 }
 
-// Targets per lane of a single-group direct sum: one below 32,768 targets (twice the waves for a
-// small sum), else two.
-inline int direct_targets_per_lane(int n_trg) { return n_trg < 32768 ? 1 : 2; }
+// Targets per lane of a direct sum in one launch.  FP64: two (half the LDS reads per pair), but one for
+// more than six outputs, whose two-target loops take 130-254 VGPRs (two or three waves per SIMD).
+// Mixed mode: one below 32,768 targets, else two (its FP32 partial sums follow the tiles of 64*T
+// targets).
+__host__ __device__ constexpr int direct_fp64_targets(int kt) { return kt > 6 ? 1 : 2; }
+inline int direct_targets_per_lane(int prec, int kt, int n_trg) {
+    return prec == 0 ? direct_fp64_targets(kt) : (n_trg < 32768 ? 1 : 2);
+}
+// Direct sums that run in one launch.  In mixed mode its FP32 sums are to be the item kernels', bit for
+// bit; three micro-kernels (double-layer PVelGrad and Laplacian, quadrupole PGradGrad) compile there
+// with another choice of which product of a dot product's first sum is fused (g0 n0 + g3 n1), 1e-8 of
+// the result apart, and keep the item kernels.  tests/test_gpu_direct_launch.py holds all others to it.
+inline bool direct_in_one_launch(int prec, int uk) { return prec == 0 || (uk != 15 && uk != 17 && uk != 22); }
 // Direct sums with at least this many sources and targets order their points (sort_points) in the
 // plan-based entries.
 constexpr int kDirectSortMin = 16384;
@@ -238,6 +264,12 @@ hipError_t launch_stage_records(int uk, int prec, const StageArgs &a, int n_copi
 hipError_t launch_items_sgpr(int uk, int prec, int T, int grid, const ItemArgs &a, const double *recs,
                              int level_min, hipStream_t s);
 hipError_t items_sgpr_occupancy(int uk, int prec, int T, int *blocks_per_cu);
+// direct sum: one launch, and a second one over the partial sums when there are several chunks
+int uker_run(int uk);
+// device memory for the chunks' partial sums of the direct-sum entries on the current device
+// (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
+int direct_partial_ptr(double **out);
+hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s);
 // equivalent / check surfaces (surface.hip)
 __host__ __device__ inline int surface_count(int p) { return 6 * (p - 1) * (p - 1) + 2; }
 void surface_host(int p, const double *c, double alpha, int depth, double *coord);

@@ -28,7 +28,9 @@
 #include <type_traits>
 
 #include "p2p_clear.hpp"
+#include "p2p_direct.hpp"
 #include "p2p_internal.hpp"
+#include "p2p_mixed.hpp"
 #include "p2p_queue.hpp"
 #include "p2p_redo.hpp"
 #include "p2p_sgpr.hpp"
@@ -96,11 +98,6 @@ template <class K> struct MixedUnroll<K, decltype((void)K::MIXED_UNROLL)> {
     static constexpr int value = K::MIXED_UNROLL;
 };
 
-// the mixed-mode source loop takes each block's first source on its own (MIXED_PEEL of the
-// micro-kernel, else not): measured on MI355X, same box, twice each: the fused PVel U-list 7.870 ->
-// 7.830 ms, the RPY U-list 39.98 -> 39.78 ms, the single-layer PVel FMM lists 6.84 -> 6.80 ms (X
-// list -1.3 %, W list +0.4 %), but the ordered Stokeslet instances 34.54 -> 34.86 ms
-template <class K, class = void> struct MixedPeel { static constexpr bool value = false; };
 // the mixed-mode source loop at one lane per target fully unrolled over a block, each source at an
 // immediate LDS offset from one base and a scheduling barrier between sources (MIXED_BLOCK_UNROLL of
 // the micro-kernel, else not): measured on MI355X, same box, twice each: the RPY U-list 41.67 ->
@@ -110,9 +107,6 @@ template <class K, class = void> struct MixedPeel { static constexpr bool value 
 template <class K, class = void> struct MixedBlockUnroll { static constexpr bool value = false; };
 template <class K> struct MixedBlockUnroll<K, decltype((void)K::MIXED_BLOCK_UNROLL)> {
     static constexpr bool value = K::MIXED_BLOCK_UNROLL;
-};
-template <class K> struct MixedPeel<K, decltype((void)K::MIXED_PEEL)> {
-    static constexpr bool value = K::MIXED_PEEL;
 };
 
 // minimum resident waves per SIMD asked of the compiler for the mixed-mode item kernel:
@@ -124,15 +118,6 @@ template <class K, class = void> struct MixedMinWaves { static constexpr int val
 template <class K> struct MixedMinWaves<K, decltype((void)K::MIXED_MIN_WAVES)> {
     static constexpr int value = K::MIXED_MIN_WAVES;
 };
-// sources per FP32 partial sum in mixed mode (a multiple of kMixedAccBlock that divides the 64-source
-// tile): MIXED_ACC_SOURCES of the micro-kernel, else kMixedAccBlock.  The path (masked / clear / far)
-// is still chosen per kMixedAccBlock sources.
-template <class K, class = void> struct MixedFlush { static constexpr int value = kMixedAccBlock; };
-template <class K> struct MixedFlush<K, decltype((void)K::MIXED_ACC_SOURCES)> {
-    static constexpr int value = K::MIXED_ACC_SOURCES;
-    static_assert(value % kMixedAccBlock == 0 && kSrcTile % value == 0, "MIXED_ACC_SOURCES");
-};
-
 template <int UK, int PREC> struct ItemMinWaves {
     static constexpr int value = (PREC != 0) ? MixedMinWaves<typename UkerOf<UK>::type>::value : 1;
 };
@@ -589,11 +574,13 @@ UkerOps make_uker_ops() {
     o.launch_sgpr = launch_sgpr_uk<UK>;
     o.occ_sgpr = occ_sgpr_uk<UK>;
     o.stage = stage_records_uk<UK>;
+    o.direct = launch_direct_uk<UK>;
     o.words[0] = RecLayout<K, 0>::WORDS;
     o.words[1] = RecLayout<K, 1>::WORDS;
     o.ks = K::KS;
     o.ks1 = K::KS1;
     o.kt = K::KT;
+    o.run = MixedFlush<K>::value;
     return o;
 }
 

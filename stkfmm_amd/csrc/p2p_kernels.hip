@@ -163,6 +163,43 @@ hipError_t launch_stage_records(int uk, int prec, const StageArgs &a, int n_copi
     return o ? o->stage(prec, a, n_copies, s) : hipErrorInvalidValue;
 }
 
+// out(perm[i], k) += scale * sum over the chunks, in chunk order, of partial[chunk][k][i]
+__global__ void __launch_bounds__(256) direct_reduce_kernel(DirectArgs a, int chunks, int kt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+    if (i >= a.n_trg)
+        return;
+    double s = 0.0;
+#pragma unroll 8
+    for (int c = 0; c < chunks; ++c)
+        s += a.partial[((long long)c * kt + k) * a.n_trg + i];
+    const long long o = a.perm ? (long long)a.perm[i] : i;
+    a.out.p[o * a.out.s + k * a.out.fs] += a.scale * s;
+}
+
+int uker_run(int uk) {
+    const UkerOps *o = uker_ops(uk);
+    return o ? o->run : -1;
+}
+
+hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s) {
+    const UkerOps *o = uker_ops(uk);
+    if (!o)
+        return hipErrorInvalidValue;
+    if (a.n_src <= 0 || a.n_trg <= 0)
+        return hipSuccess;
+    a.ls = l.ls;
+    a.unit = l.unit;
+    a.tail_begin = l.tail_begin;
+    a.tail_ls = l.tail_ls;
+    a.chunk_tiles = l.chunk_tiles;
+    const hipError_t e = o->direct(prec, l.T, a, l, s);
+    if (e != hipSuccess || l.chunks == 1)
+        return e;
+    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 255) / 256), (unsigned)o->kt), dim3(256), 0, s,
+                       a, l.chunks, o->kt);
+    return hipGetLastError();
+}
+
 int record_words(int uk, int prec) {
     const UkerOps *o = uker_ops(uk);
     return (o && (prec == 0 || prec == 1)) ? o->words[prec] : -1;
