@@ -633,7 +633,8 @@ def wall_images(args, torch, S, W):
     targets in z in (0, 0.5) above the wall z = 0: Stokes (7 constituent direct sums of n x m pairs:
     the Stokeslet, LapPGrad and LapPGradGrad over originals + images, the dipole sum over images) and
     RPY (10: RPY, LapPGradGrad, LapPGrad and dipole sums over originals + images, the dipole and
-    quadrupole gradient sums over images); a pair is one evaluation in one constituent sum."""
+    quadrupole gradient sums over images); a pair is one evaluation in one constituent sum (the library
+    evaluates a source and its image as one pair formula, the whole system per source and target)."""
     dev = torch.device("cuda:0")
     n = 65_536
     g = np.random.default_rng(31)

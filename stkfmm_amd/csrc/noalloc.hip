@@ -217,8 +217,8 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
         a.scale = uker_scale(uk);
         a.n_src = nSrc;
         a.n_trg = nTrg;
-        const DirectLayout l = direct_layout(precision, direct_targets_per_lane(precision, kt, nTrg), kt, uker_run(uk), nSrc,
-                                             nTrg, n_cu);
+        const DirectLayout l = direct_layout_uk(uk, precision, direct_targets_per_lane(precision, kt, nTrg), nSrc, nTrg,
+                                                n_cu);
         if ((e = launch_direct(uk, precision, a, l, s)) != hipSuccess)
             return fail(STKFMM_ERR_HIP, "no-alloc direct sum: launch failed");
         return STKFMM_OK;

@@ -677,8 +677,8 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         p->dn_trg = grp_trg_end[0] - p->dt_begin;
         p->ds_begin = rng_src_begin[r0];
         p->dn_src = rng_src_end[r0] - p->ds_begin;
-        p->dlayout = direct_layout(precision, precision == STKFMM_PREC_FP64 ? direct_fp64_targets(p->KT) : T, p->KT, uker_run(uk), p->dn_src,
-                                   p->dn_trg, n_cu);
+        p->dlayout = direct_layout_uk(uk, precision, precision == STKFMM_PREC_FP64 ? direct_fp64_targets(p->KT) : T,
+                                      p->dn_src, p->dn_trg, n_cu);
         if (p->dlayout.chunks > 1) {
             const hipError_t e = hipMalloc((void **)&p->d_partial,
                                            sizeof(double) * p->dlayout.chunks * p->KT * (size_t)p->dn_trg);
@@ -1056,10 +1056,9 @@ int direct_plan(int uk, int prec, int n_src, int n_trg, stkfmm_plan **out) {
 // grow-only device buffers for the host-pointer entries
 struct Workspace {
     int device = -1;
-    // slot 0: host-pointer entries (inputs and output, packed); slots 1-3: unused; slot 4: adjoint
-    // partial sums; slot 5: wall images
-    double *buf[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    size_t cap[6] = {0, 0, 0, 0, 0, 0};
+    // slot 0: host-pointer entries (inputs and output, packed); slot 1: adjoint partial sums
+    double *buf[2] = {nullptr, nullptr};
+    size_t cap[2] = {0, 0};
 };
 std::vector<Workspace> g_ws;
 
@@ -1101,8 +1100,7 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
         double *partial = nullptr;
         if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
             return rc;
-        const DirectLayout l = direct_layout(prec, direct_targets_per_lane(prec, kt, n_trg), kt, uker_run(uk), n_src, n_trg,
-                                             n_cu);
+        const DirectLayout l = direct_layout_uk(uk, prec, direct_targets_per_lane(prec, kt, n_trg), n_src, n_trg, n_cu);
         return enqueue_direct(uk, prec, l, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
                               DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, partial, s);
     }
@@ -1217,60 +1215,28 @@ extern "C" int stkfmm_p2p_eval_device(unsigned kernel, unsigned p2p, int precisi
 // ---- wall images (StkWallFMM, Lib/src/StkWallFMM.cpp:154-292) ----------------------------------------
 
 namespace {
-// the constituent direct sums of StkWallFMM::evalStokes / evalRPY, with the layouts of wall.hip
-int wall_device(unsigned kernel, int prec, int n, const double *sc, const double *sv, int m, const double *tc,
-                double *tv, hipStream_t s) {
-    const size_t N = (size_t)n, M = (size_t)m;
-    double *w = nullptr;
-    int rc;
-    if (kernel == STKFMM_KERNEL_Stokes) {
-        if ((rc = ws_get(5, 6 * N + 6 * N + 2 * N + 3 * N + 2 * N + 17 * M, &w)))
-            return rc;
-        WallStokes L;
-        L.c2 = w;
-        L.vS = L.c2 + 6 * N;
-        L.vL1 = L.vS + 6 * N;
-        L.vD = L.vL1 + 2 * N;
-        L.vL2 = L.vD + 3 * N;
-        L.oS = L.vL2 + 2 * N;
-        L.oL1D = L.oS + 3 * M;
-        L.oL2 = L.oL1D + 4 * M;
-        HIP_TRY(launch_wall_prep_stokes(n, sc, sv, L, s), "wall prep launch");
-        HIP_TRY(launch_wall_zero(L.oS, (long long)(17 * M), s), "wall zero launch");
-        const double *cimg = L.c2 + 3 * N;
-        if ((rc = eval_device_uk(STKFMM_UKER_STOKES_VEL, prec, 2 * n, L.c2, L.vS, m, tc, L.oS, s)) ||
-            (rc = eval_device_uk(STKFMM_UKER_LAPLACE_PGRAD, prec, 2 * n, L.c2, L.vL1, m, tc, L.oL1D, s)) ||
-            (rc = eval_device_uk(STKFMM_UKER_LAPLACE_DIPOLEPGRAD, prec, n, cimg, L.vD, m, tc, L.oL1D, s)) ||
-            (rc = eval_device_uk(STKFMM_UKER_LAPLACE_PGRADGRAD, prec, 2 * n, L.c2, L.vL2, m, tc, L.oL2, s)))
-            return rc;
-        HIP_TRY(launch_wall_assemble_stokes(m, tc, L, tv, s), "wall assemble launch");
-        return STKFMM_OK;
+// one direct sum of source-and-image pairs (wall.hip)
+int wall_device(unsigned kernel, const double *sc, const double *sv, int n, const double *tc, double *tv, int m,
+                hipStream_t s) {
+    int n_cu = 0, rc;
+    double *partial = nullptr;
+    if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
+        return rc;
+    const int ks = kernel == STKFMM_KERNEL_Stokes ? 3 : 4, kt = kernel == STKFMM_KERNEL_Stokes ? 3 : 6;
+    // target slabs keep the launch inside its index range
+    const int slab = 1 << 29;
+    for (long long t0 = 0; t0 < m; t0 += slab) {
+        DirectArgs a{};
+        a.sc = DArr{sc, 3, 1};
+        a.v1 = a.v2 = DArr{sv, ks, 1};
+        a.tc = DArr{tc + 3 * t0, 3, 1};
+        a.out = OArr{tv + kt * t0, kt, 1};
+        a.partial = partial;
+        a.scale = uker_scale(STKFMM_UKER_STOKES_VEL);
+        a.n_src = n;
+        a.n_trg = (int)std::min<long long>(slab, m - t0);
+        HIP_TRY(launch_wall(kernel == STKFMM_KERNEL_RPY, a, n_cu, s), "wall images launch");
     }
-    if ((rc = ws_get(5, 6 * N + 8 * N + 2 * N + 3 * N + 2 * N + 6 * N + 9 * N + 30 * M, &w)))
-        return rc;
-    WallRpy L;
-    L.c2 = w;
-    L.vR = L.c2 + 6 * N;
-    L.vLS = L.vR + 8 * N;
-    L.vLD = L.vLS + 2 * N;
-    L.vLSZ = L.vLD + 3 * N;
-    L.vLDZ = L.vLSZ + 2 * N;
-    L.vQ = L.vLDZ + 6 * N;
-    L.oR = L.vQ + 9 * N;
-    L.oSD = L.oR + 6 * M;
-    L.oSDZ = L.oSD + 10 * M;
-    L.oQ = L.oSDZ + 4 * M;
-    HIP_TRY(launch_wall_prep_rpy(n, sc, sv, L, s), "wall prep launch");
-    HIP_TRY(launch_wall_zero(L.oR, (long long)(30 * M), s), "wall zero launch");
-    const double *cimg = L.c2 + 3 * N;
-    if ((rc = eval_device_uk(STKFMM_UKER_RPY_ULAPU, prec, 2 * n, L.c2, L.vR, m, tc, L.oR, s)) ||
-        (rc = eval_device_uk(STKFMM_UKER_LAPLACE_PGRADGRAD, prec, 2 * n, L.c2, L.vLS, m, tc, L.oSD, s)) ||
-        (rc = eval_device_uk(STKFMM_UKER_LAPLACE_DIPOLEPGRADGRAD, prec, n, cimg, L.vLD, m, tc, L.oSD, s)) ||
-        (rc = eval_device_uk(STKFMM_UKER_LAPLACE_PGRAD, prec, 2 * n, L.c2, L.vLSZ, m, tc, L.oSDZ, s)) ||
-        (rc = eval_device_uk(STKFMM_UKER_LAPLACE_DIPOLEPGRAD, prec, 2 * n, L.c2, L.vLDZ, m, tc, L.oSDZ, s)) ||
-        (rc = eval_device_uk(STKFMM_UKER_LAPLACE_QUADPGRADGRAD, prec, n, cimg, L.vQ, m, tc, L.oQ, s)))
-        return rc;
-    HIP_TRY(launch_wall_assemble_rpy(m, tc, L, tv, s), "wall assemble launch");
     return STKFMM_OK;
 }
 
@@ -1303,8 +1269,7 @@ extern "C" int stkfmm_wall_eval_device(unsigned kernel, int precision, int nSL, 
     if (!d_srcCoord || !d_srcValue || !d_trgCoord || !d_trgValue)
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
     std::lock_guard<std::mutex> lk(g_mu);
-    return wall_device(kernel, precision, nSL, d_srcCoord, d_srcValue, nTrg, d_trgCoord, d_trgValue,
-                       (hipStream_t)stream);
+    return wall_device(kernel, d_srcCoord, d_srcValue, nSL, d_trgCoord, d_trgValue, nTrg, (hipStream_t)stream);
 }
 
 extern "C" int stkfmm_wall_evaluate(unsigned kernel, int precision, int nSL, const double *srcCoord,
@@ -1320,7 +1285,7 @@ extern "C" int stkfmm_wall_evaluate(unsigned kernel, int precision, int nSL, con
     std::lock_guard<std::mutex> lk(g_mu);
     return host_roundtrip(ks, kt, nSL, srcCoord, srcValue, nTrg, trgCoord, trgValue,
                           [&](const double *d_sc, const double *d_sv, const double *d_tc, double *d_tv) {
-                              return wall_device(kernel, precision, nSL, d_sc, d_sv, nTrg, d_tc, d_tv, nullptr);
+                              return wall_device(kernel, d_sc, d_sv, nSL, d_tc, d_tv, nTrg, nullptr);
                           });
 }
 
@@ -1447,7 +1412,7 @@ extern "C" int stkfmm_p2p_vjp_device(int uker, int precision, int nSrc, const do
     std::lock_guard<std::mutex> lk(g_mu);
     double *partial = nullptr;
     const size_t need = (size_t)l.n_chunks * 3 * nTrg + (size_t)l.n_blocks * (3 + ks) * nSrc;
-    if ((rc = ws_get(4, std::max<size_t>(need, 1), &partial)))
+    if ((rc = ws_get(1, std::max<size_t>(need, 1), &partial)))
         return rc;
     VjpArgs a{d_srcCoord, d_srcValue, d_trgCoord, d_w, nSrc, nTrg, uker_scale(uker),
               d_g_src_value, d_g_src_coord, d_g_trg_coord};

@@ -42,6 +42,10 @@ template <class K, int PREC> struct DirectLds {
     static constexpr int WORDS = (PREC == 0) ? (3 + KL) * kSrcTile : 3 * kSrcTile + kSrcTile * KLP / 2;
 };
 
+// pairs of a source and its wall image (wall_pairs.hpp), which take the heights over the wall as well
+template <class K, class = void> struct IsWallPair { static constexpr bool value = false; };
+template <class K> struct IsWallPair<K, decltype((void)K::WALL)> { static constexpr bool value = K::WALL; };
+
 // LDS written by some lanes of a wave is read by others of the same wave only: the LDS keeps a wave's
 // accesses in order, so it is enough that the compiler does
 __device__ __forceinline__ void wave_lds_fence() {
@@ -66,7 +70,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
     float *const rows = reinterpret_cast<float *>(sm + 3 * kSrcTile);
 
     // this workgroup's targets, and how its lanes share them
-    int ls = a.ls, tb = (int)blockIdx.x * a.unit, te = min(tb + a.unit, a.n_trg);
+    int ls = a.ls, tb = (int)blockIdx.x * a.unit, te = tb + min(a.unit, a.n_trg - tb);
     bool runs = PREC != 0; // lanes share a target by whole FP32 runs
     if (PREC != 0 && a.tail_ls > 0) {
         if ((int)blockIdx.x == (int)gridDim.x - 1) {
@@ -84,7 +88,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
     double tx[T], ty[T], tz[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const long long i = min(tb + slot + slots * t, te - 1);
+        const long long i = tb + min(slot + slots * t, te - tb - 1);
         tx[t] = a.tc.p[i * a.tc.s];
         ty[t] = a.tc.p[i * a.tc.s + a.tc.fs];
         tz[t] = a.tc.p[i * a.tc.s + 2 * a.tc.fs];
@@ -104,7 +108,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
 
     double c[3], vin[KS];
     auto fetch = [&](int st) {
-        const long long s = min(st * kSrcTile + lane, a.n_src - 1);
+        const long long s = min((long long)st * kSrcTile + lane, (long long)a.n_src - 1);
 #pragma unroll
         for (int d = 0; d < 3; ++d)
             c[d] = a.sc.p[s * a.sc.s + d * a.sc.fs];
@@ -119,11 +123,15 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
         for (int k = 0; k < KL; ++k)
             f[k] = sm[(3 + k) * kSrcTile + j];
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-            eval_pair<K, true>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
+        for (int t = 0; t < T; ++t) {
+            if constexpr (IsWallPair<K>::value)
+                K::eval_wall(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, tz[t] + sz, tz[t], f);
+            else
+                eval_pair<K, true>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
+        }
     };
     float part[T][KT];
-    auto pair32 = [&](int j) {
+    auto pair32 = [&](auto j) { // (generic: instantiated in mixed mode only)
         const double sx = sm[j], sy = sm[kSrcTile + j], sz = sm[2 * kSrcTile + j];
         float f[KL];
 #pragma unroll
@@ -160,6 +168,8 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
         const int n = min(kSrcTile, a.n_src - st * kSrcTile);
         double vst[KL];
         stage_for<K, PREC>(vin, vst);
+        if constexpr (IsWallPair<K>::value)
+            K::stage_height(c[2], vst);
         wave_lds_fence(); // every lane has read the previous tile
 #pragma unroll
         for (int d = 0; d < 3; ++d)

@@ -26,17 +26,23 @@ struct DirectLayout {
 // (kAlone).  The partial sums of c chunks cost a second launch and their reads, kReduce + c kChunk.  Fitted
 // to a sweep of ls, chunks and waves over 11 shapes in each precision; the cut taken is within 15 % of
 // the sweep's best (for instance 8192^2 LapPGrad FP64 54 us, best 53; 9,000 x 1,000 PVel 19 us, best 18).
-inline DirectLayout direct_layout(int prec, int T, int kt, int run, int n_src, int n_trg, int n_cu) {
+struct DirectCost {
+    double pair;   // cycles of a pair in one lane
+    int max_waves; // waves per workgroup, at most: half of kDirectWaves where registers leave two or three
+                   // waves per SIMD (more than six outputs: 120-156 VGPRs), so that workgroups pack
+    int overlap;   // workgroups of a CU whose set-up (targets, the waves' sums) overlaps others' pairs
+};
+inline DirectCost direct_cost(int prec, int kt) {
+    return DirectCost{prec == 0 ? 50.0 + 15.0 * kt : 50.0 + 8.0 * kt, kt > 6 ? kDirectWaves / 2 : kDirectWaves,
+                      kt <= 4 ? 4 : (kt <= 6 ? 1 : 2)};
+}
+inline DirectLayout direct_layout(int prec, int T, const DirectCost &cost, int run, int n_src, int n_trg, int n_cu) {
     const int TT = kWave * T;
-    const long long stiles = (n_src + kSrcTile - 1) / kSrcTile;
+    const long long stiles = ((long long)n_src + kSrcTile - 1) / kSrcTile;
     DirectLayout best{};
     double best_t = -1.0;
     const int ls_max = (prec == 0) ? 4 : (run >= 64 ? 0 : (run == 32 ? 1 : 2));
-    const double pair = (prec == 0 ? 50.0 + 15.0 * kt : 50.0 + 8.0 * kt);
     const double kStage = 800.0, kSetup = 4000.0, kReduce = 8000.0, kChunk = 250.0, kAlone = 3.0;
-    // workgroups of a CU whose set-up (targets, the waves' sums) overlaps others' pairs: by registers
-    const int overlap = kt <= 4 ? 4 : (kt <= 6 ? 1 : 2);
-    const int max_waves = kt > 6 ? kDirectWaves / 2 : kDirectWaves; // 120-156 VGPRs: finer packing
     for (int ls = 0; ls <= ls_max; ++ls) {
         DirectLayout l{};
         l.T = T;
@@ -57,14 +63,15 @@ inline DirectLayout direct_layout(int prec, int T, int kt, int run, int n_src, i
                 break;
             l.chunk_tiles = (int)((stiles + c - 1) / c);
             l.chunks = (int)((stiles + l.chunk_tiles - 1) / l.chunk_tiles);
-            l.waves = max_waves;
+            l.waves = cost.max_waves;
             while (l.waves > 1 && l.waves / 2 >= l.chunk_tiles)
                 l.waves /= 2;
             const double rounds = (double)((l.chunk_tiles + l.waves - 1) / l.waves);
-            const double wave_t = rounds * (kStage + (kWave >> ls) * T * pair);
+            const double wave_t = rounds * (kStage + (kWave >> ls) * T * cost.pair);
             const long long wgs = ((long long)l.units * l.chunks + n_cu - 1) / n_cu;
             const double per_simd = (double)(wgs * l.waves) / 4.0; // waves a SIMD has to run
-            const double t = kSetup * (double)((wgs + overlap - 1) / overlap) + wave_t * (per_simd > kAlone ? per_simd + 0.25 : kAlone + 0.25) +
+            const double t = kSetup * (double)((wgs + cost.overlap - 1) / cost.overlap) +
+                             wave_t * ((per_simd > kAlone ? per_simd : kAlone) + 0.25) +
                              (l.chunks > 1 ? kReduce + kChunk * l.chunks : 0.0);
             if (best_t < 0.0 || t < best_t) {
                 best_t = t;
@@ -73,6 +80,11 @@ inline DirectLayout direct_layout(int prec, int T, int kt, int run, int n_src, i
         }
     }
     return best;
+}
+
+// the layout of micro-kernel uk's direct sum, T targets per lane
+inline DirectLayout direct_layout_uk(int uk, int prec, int T, int n_src, int n_trg, int n_cu) {
+    return direct_layout(prec, T, direct_cost(prec, uker_kt(uk)), uker_run(uk), n_src, n_trg, n_cu);
 }
 
 } // namespace stkp2p

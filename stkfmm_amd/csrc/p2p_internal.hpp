@@ -100,6 +100,7 @@ struct DirectArgs {
     int ls, unit, tail_begin, tail_ls, chunk_tiles; // DirectLayout
 };
 struct DirectLayout;
+void direct_args_layout(DirectArgs &a, const DirectLayout &l);
 // the chunks' partial sums hold at most this many targets' outputs (16 MiB at 16 outputs)
 constexpr long long kDirectPartialTargets = 131072;
 
@@ -269,27 +270,15 @@ int uker_run(int uk);
 // device memory for the chunks' partial sums of the direct-sum entries on the current device
 // (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
 int direct_partial_ptr(double **out);
+hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s);
 hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s);
 // equivalent / check surfaces (surface.hip)
 __host__ __device__ inline int surface_count(int p) { return 6 * (p - 1) * (p - 1) + 2; }
 void surface_host(int p, const double *c, double alpha, int depth, double *coord);
 hipError_t launch_box_surfaces(int p, double alpha, int n_boxes, const double *corner, const int *level, double *out,
                                hipStream_t s);
-// wall image system (wall.hip): device views of the workspace of one evaluation.  n sources
-// (2n with images: [originals; images]), m targets; v* are source values, o* accumulated outputs.
-struct WallStokes {
-    double *c2, *vS, *vL1, *vD, *vL2; // [2n*3], [2n*3], [2n], [n*3] (at the images), [2n]
-    double *oS, *oL1D, *oL2;          // [m*3], [m*4], [m*10]
-};
-struct WallRpy {
-    double *c2, *vR, *vLS, *vLD, *vLSZ, *vLDZ, *vQ; // [2n*3],[2n*4],[2n],[n*3],[2n],[2n*3],[n*9]
-    double *oR, *oSD, *oSDZ, *oQ;                   // [m*6], [m*10], [m*4], [m*10]
-};
-hipError_t launch_wall_prep_stokes(int n, const double *sc, const double *sv, const WallStokes &w, hipStream_t s);
-hipError_t launch_wall_prep_rpy(int n, const double *sc, const double *sv, const WallRpy &w, hipStream_t s);
-hipError_t launch_wall_zero(double *p, long long n, hipStream_t s);
-hipError_t launch_wall_assemble_stokes(int m, const double *tc, const WallStokes &w, double *out, hipStream_t s);
-hipError_t launch_wall_assemble_rpy(int m, const double *tc, const WallRpy &w, double *out, hipStream_t s);
+// wall image system (wall.hip): a direct sum of source-and-image pairs (a.partial: direct_partial_ptr)
+hipError_t launch_wall(bool rpy, DirectArgs a, int n_cu, hipStream_t s);
 // adjoint work decomposition: T targets per lane; the grid is n_blocks target blocks (of
 // trg_tiles_per_block tiles of 64 T targets) x n_chunks source chunks (of src_tiles_per_chunk tiles of
 // 64 sources); partial holds n_chunks * 3 * n_trg + n_blocks * (3 + KS) * n_src doubles

@@ -181,23 +181,31 @@ int uker_run(int uk) {
     return o ? o->run : -1;
 }
 
+void direct_args_layout(DirectArgs &a, const DirectLayout &l) {
+    a.ls = l.ls;
+    a.unit = l.unit;
+    a.tail_begin = l.tail_begin;
+    a.tail_ls = l.tail_ls;
+    a.chunk_tiles = l.chunk_tiles;
+}
+
+hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s) {
+    if (chunks == 1)
+        return hipSuccess;
+    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 255) / 256), (unsigned)kt), dim3(256), 0, s, a,
+                       chunks, kt);
+    return hipGetLastError();
+}
+
 hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s) {
     const UkerOps *o = uker_ops(uk);
     if (!o)
         return hipErrorInvalidValue;
     if (a.n_src <= 0 || a.n_trg <= 0)
         return hipSuccess;
-    a.ls = l.ls;
-    a.unit = l.unit;
-    a.tail_begin = l.tail_begin;
-    a.tail_ls = l.tail_ls;
-    a.chunk_tiles = l.chunk_tiles;
+    direct_args_layout(a, l);
     const hipError_t e = o->direct(prec, l.T, a, l, s);
-    if (e != hipSuccess || l.chunks == 1)
-        return e;
-    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 255) / 256), (unsigned)o->kt), dim3(256), 0, s,
-                       a, l.chunks, o->kt);
-    return hipGetLastError();
+    return e != hipSuccess ? e : launch_direct_reduce(a, l.chunks, o->kt, s);
 }
 
 int record_words(int uk, int prec) {

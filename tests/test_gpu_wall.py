@@ -102,3 +102,24 @@ def test_wall_repeated_calls_with_other_sizes():
         S.wall_device(S.KERNEL.RPY, to_dev(x), to_dev(np.ascontiguousarray(f)), to_dev(t), out)
         l2, mx = O.max_error(host(out), O.wall(16, x, f, t))
         assert mx < FP64_TOL or np.all(O.wall(16, x, f, t) == 0)
+
+
+@pytest.mark.parametrize("kernel", [S.KERNEL.Stokes, S.KERNEL.RPY])
+@pytest.mark.parametrize("ns,nt", [(1, 64), (63, 65), (129, 17), (5000, 3), (20, 4100), (2500, 700)])
+def test_wall_sizes_at_the_edges_of_the_launch(kernel, ns, nt):
+    """One tile more or less, source chunks, lanes sharing targets; sources on the wall (which coincide with
+    their images) and targets at them."""
+    say(f"wall edges kernel={int(kernel)} ns={ns} nt={nt}")
+    x, f, t = problem(kernel, ns + nt, ns=ns, nt=nt)
+    k = max(1, ns // 7)
+    x[-k:, 2] = 0.0
+    t[-1] = x[-1]
+    kt = 3 if kernel == S.KERNEL.Stokes else 6
+    ref = O.wall(int(kernel), x, f, t)
+    rev = O.wall(int(kernel), x[::-1], f[::-1], t)
+    _, cond = O.max_error(rev, ref)  # the reference's own conditioning: its sums cancel near the wall
+    out = zeros(nt, kt)
+    S.wall_device(kernel, to_dev(x), to_dev(np.ascontiguousarray(f)), to_dev(t), out)
+    l2, mx = O.max_error(host(out), ref)
+    bound = max(4 * cond, FP64_TOL)
+    assert l2 < bound and mx < bound, (l2, mx, cond)
