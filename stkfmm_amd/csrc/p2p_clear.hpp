@@ -28,6 +28,31 @@ __device__ __forceinline__ void eval_pair(R *u, R dx, R dy, R dz, const R *f) {
         K::template eval<R>(u, dx, dy, dz, f);
 }
 
+// one pair into the accumulators of precision PREC (AccCount): the FP64 form with accumulators of its own
+// where the micro-kernel has one, else its outputs
+template <class K, int PREC, bool MASK, class R>
+__device__ __forceinline__ void eval_acc(R *u, R dx, R dy, R dz, const R *f) {
+    if constexpr (PREC == 0 && HasEval64<K>::value)
+        K::template eval64<MASK>(u, dx, dy, dz, f);
+    else
+        eval_pair<K, MASK>(u, dx, dy, dz, f);
+}
+// precision PREC has an unmasked form
+template <class K, int PREC> struct HasClearForm {
+    static constexpr bool value = HasUnmaskedEval<K>::value || (PREC == 0 && HasEval64<K>::value);
+};
+// a target's outputs (before post()) from its accumulators
+template <class K, int PREC>
+__device__ __forceinline__ void finish_acc(const double *acc, double *out) {
+    if constexpr (PREC == 0 && HasEval64<K>::value) {
+        K::finish64(acc, out);
+    } else {
+#pragma unroll
+        for (int k = 0; k < K::KT; ++k)
+            out[k] = acc[k];
+    }
+}
+
 // a wave-uniform double held in scalar registers (every lane has the same value)
 __device__ __forceinline__ double uniform_f64(double v) {
     const unsigned long long b = __builtin_bit_cast(unsigned long long, v);

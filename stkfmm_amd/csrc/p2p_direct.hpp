@@ -58,6 +58,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
     using K = typename UkerOf<UK>::type;
     using L = DirectLds<K, PREC>;
     constexpr int KL = L::KL, KLP = L::KLP, KT = K::KT, KS = K::KS, KS1 = K::KS1, TT = kWave * T;
+    constexpr int NA = AccCount<K, PREC>::value;
     constexpr int RUN = (PREC == 0) ? kSrcTile : MixedFlush<K>::value;
     // a run's first source on its own where the item kernels take it so: its products then start the
     // sums, which decides which of them is rounded (f/r + r b: one FMA of either product)
@@ -93,11 +94,11 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
         ty[t] = a.tc.p[i * a.tc.s + a.tc.fs];
         tz[t] = a.tc.p[i * a.tc.s + 2 * a.tc.fs];
     }
-    double acc[T][KT];
+    double acc[T][NA];
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int k = 0; k < KT; ++k)
+        for (int k = 0; k < NA; ++k)
             acc[t][k] = 0.0;
 
     // runs start at g0, g0 + gs, ... of a tile; a lane takes sources j0, j0 + js, ... of each
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
             if constexpr (IsWallPair<K>::value)
                 K::eval_wall(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, tz[t] + sz, tz[t], f);
             else
-                eval_pair<K, true>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
+                eval_acc<K, PREC, true>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
         }
     };
     float part[T][KT];
@@ -282,8 +283,12 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int k = 0; k < KT; ++k)
+            for (int k = 0; k < NA; ++k)
                 acc[t][k] += __shfl_xor(acc[t][k], off);
+    double out[T][KT];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+        finish_acc<K, PREC>(acc[t], out[t]);
     constexpr int KG0 = L::WORDS / TT, KG = KG0 < KT ? KG0 : KT;
     static_assert(KG >= 1, "the waves' sums fit the staging memory");
     const int lgu = 6 - ls + (T == 2 ? 1 : 0); // log2 of the unit's target slots
@@ -296,7 +301,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
                 if (k0 + q < KT)
 #pragma unroll
                     for (int t = 0; t < T; ++t)
-                        smem[(wave * KG + q) * TT + slot + slots * t] = acc[t][k0 + q < KT ? k0 + q : 0];
+                        smem[(wave * KG + q) * TT + slot + slots * t] = out[t][k0 + q < KT ? k0 + q : 0];
         }
         __syncthreads();
         const int nk = (KT - k0 < KG) ? KT - k0 : KG;

@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(kWave) STKP2P_ITEM_ATTR
 __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_kernel(ItemArgs a) {
     using K = typename UkerOf<UK>::type;
     constexpr int KL = StagedCount<K, PREC>::value, KT = K::KT, KS = K::KS, KS1 = K::KS1;
-    constexpr int TT = kWave * T;
+    constexpr int TT = kWave * T, NA = AccCount<K, PREC>::value;
 
     // FP64: values as [KL][tile] (two consecutive sources per 16-byte read);
     // mixed: FP32 values as 16-byte aligned rows [tile][KLP] (one source per few 16-byte reads,
@@ -188,7 +188,7 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
             }
         }
         // target box for the unmasked shortcut on source tiles clear of it (p2p_clear.hpp)
-        constexpr bool CLEAR = HasUnmaskedEval<K>::value && !HILO;
+        constexpr bool CLEAR = HasClearForm<K, PREC>::value && !HILO;
         TargetBox<PREC> box;
         if constexpr (CLEAR)
             box.build(tx, ty, tz);
@@ -211,11 +211,11 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
                 tfz[t] = (float)(tz[t] - fc[2]);
             }
         }
-        double acc[T][KT];
+        double acc[T][NA];
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int k = 0; k < KT; ++k)
+            for (int k = 0; k < NA; ++k)
                 acc[t][k] = 0.0;
 
         for (int r = item.rng_begin; r < item.rng_end; ++r) {
@@ -324,7 +324,7 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
                                 f[k] = s_vd[k][j];
 #pragma unroll
                             for (int t = 0; t < T; ++t)
-                                eval_pair<K, MASK>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
+                                eval_acc<K, PREC, MASK>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
                         };
                         if (T == 1 && !STR && je - jb == kSrcTile) {
                             // a whole tile at one target per lane: a fixed trip count, so the
@@ -471,9 +471,13 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
 #pragma unroll
             for (int t = 0; t < T; ++t)
 #pragma unroll
-                for (int k = 0; k < KT; ++k)
+                for (int k = 0; k < NA; ++k)
                     acc[t][k] += __shfl_xor(acc[t][k], off);
         }
+        double out[T][KT];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            finish_acc<K, PREC>(acc[t], out[t]);
         double *dst = a.partial + (long long)item.slot * KT * TT;
 #pragma unroll
         for (int k = 0; k < KT; ++k) {
@@ -482,7 +486,7 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
             for (int t = 0; t < T; ++t) {
                 const int i = slot0 + tstride * t;
                 if (sub == 0 && i < item.trg_count)
-                    dst[(long long)k * TT + i] = acc[t][k] * osc;
+                    dst[(long long)k * TT + i] = out[t][k] * osc;
             }
         }
     }

@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
     using K = typename UkerOf<UK>::type;
     using L = RecLayout<K, PREC>;
     constexpr int KL = L::KL, KT = K::KT;
-    constexpr int TT = kWave * T;
+    constexpr int TT = kWave * T, NA = AccCount<K, PREC>::value;
     const int lane = threadIdx.x;
     ItemCursor cur(a);
     for (;;) {
@@ -110,15 +110,15 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
             ty[t] = a.tc.p[idx * a.tc.s + a.tc.fs] * lam;
             tz[t] = a.tc.p[idx * a.tc.s + 2 * a.tc.fs] * lam;
         }
-        constexpr bool CLEAR = HasUnmaskedEval<K>::value;
+        constexpr bool CLEAR = HasClearForm<K, PREC>::value;
         TargetBox<PREC> box;
         if constexpr (CLEAR)
             box.build(tx, ty, tz);
-        double acc[T][KT];
+        double acc[T][NA];
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int k = 0; k < KT; ++k)
+            for (int k = 0; k < NA; ++k)
                 acc[t][k] = 0.0;
 
         // one source record against the lane's T targets; P is the record pointer type (scalar
@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
                 f[k] = p[3 + k];
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                eval_pair<K, MASK>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
+                eval_acc<K, PREC, MASK>(acc[t], tx[t] - sx, ty[t] - sy, tz[t] - sz, f);
         };
 
         for (int r = item.rng_begin; r < item.rng_end; ++r) {
@@ -238,9 +238,13 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
 #pragma unroll
             for (int t = 0; t < T; ++t)
 #pragma unroll
-                for (int k = 0; k < KT; ++k)
+                for (int k = 0; k < NA; ++k)
                     acc[t][k] += __shfl_xor(acc[t][k], off);
         }
+        double out[T][KT];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            finish_acc<K, PREC>(acc[t], out[t]);
         double *dst = a.partial + (long long)item.slot * KT * TT;
 #pragma unroll
         for (int k = 0; k < KT; ++k) {
@@ -249,7 +253,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
             for (int t = 0; t < T; ++t) {
                 const int i = slot0 + tstride * t;
                 if (sub == 0 && i < item.trg_count)
-                    dst[(long long)k * TT + i] = acc[t][k] * osc;
+                    dst[(long long)k * TT + i] = out[t][k] * osc;
             }
         }
     }

@@ -20,6 +20,7 @@
 //         x_src; M = false for pairs known to have r2 > 0 (no coincidence mask),
 //   post(k) constant factor applied to accumulated output k once per work item (so that per-pair
 //         constants such as the 2 of the pressure leave the inner loop),
+//   ACC64, eval64, finish64 (some): an FP64 form with accumulators of its own (HasEval64),
 //   UNMASKED_EVAL (true here: eval<R, false> exists).
 // The hot kernels (Stokeslet, PVel single/double/fused, regularised Stokeslet, RPY, Laplace PGrad)
 // evaluate the reference expression in an equivalent form with fewer operations (common factors
@@ -165,6 +166,26 @@ __host__ __device__ constexpr double post_for(int k) {
         return K::post(k);
 }
 
+// FP64 pair form with accumulators of its own: micro-kernels that declare ACC64 accumulate ACC64 sums per
+// target with eval64<M>(a, dx, dy, dz, f) (M = false: pairs known to have r2 > 0) and turn them into the
+// outputs (before post()) once per target and work item with finish64(a, out).  It lets terms common to
+// several outputs be summed once: symmetric and antisymmetric halves of a tensor, the multiple of the
+// unit matrix in its diagonal, constant factors.  eval<double> is then one pair through both.
+template <class K, class = void> struct HasEval64 { static constexpr bool value = false; };
+template <class K> struct HasEval64<K, decltype((void)K::ACC64)> { static constexpr bool value = true; };
+template <class K, int PREC, class = void> struct AccCount { static constexpr int value = K::KT; };
+template <class K> struct AccCount<K, 0, decltype((void)K::ACC64)> { static constexpr int value = K::ACC64; };
+template <class K>
+__device__ inline void eval_by_acc64(double *u, double dx, double dy, double dz, const double *f) {
+    double a[K::ACC64], o[K::KT];
+    for (int k = 0; k < K::ACC64; ++k)
+        a[k] = 0.0;
+    K::template eval64<true>(a, dx, dy, dz, f);
+    K::finish64(a, o);
+    for (int k = 0; k < K::KT; ++k)
+        u[k] += o[k];
+}
+
 template <class K, int PREC>
 __host__ __device__ inline void stage_for(const double *in, double *o) {
     if constexpr (StagesByPrecision<K>::value)
@@ -271,15 +292,54 @@ struct UkLaplaceDipolePGrad {
 //   p = q/r,  grad p = -q r/r^3,  grad grad p_ij = q (3 r_i r_j - r^2 delta_ij)/r^5.
 // Unit-direction form (s = 1/r, n = r s): grad p = -(q s^3) r,  grad grad p_ij = q s^3 (3 n_i n_j -
 // delta_ij) -- no power above s^3 (the literal 1/r^5 overflows FP32 below r ~ 2e-8).
+// FP64: w = 2/r, A = (q/2) w, sv = A w^2 = 4 q/r^3, K = sv w^2 = 16 q/r^5; accumulators p, sv r (grad, -1/4),
+// sv (the diagonal's -1/4, summed once), K r_i r_j (diagonal and off-diagonal, 3/16).
 struct UkLaplacePGradGrad {
-    static constexpr int KS = 1, KS1 = 1, KL = 1, KT = 10;
-    static constexpr bool UNMASKED_EVAL = true;
+    static constexpr int KS = 1, KS1 = 1, KL = 1, KT = 10, ACC64 = 11;
+    static constexpr bool UNMASKED_EVAL = true, STAGE_BY_PRECISION = true;
     static constexpr unsigned SRC_SCALE_MASK = 0u;
     __host__ __device__ static constexpr int deg(int k) { return k == 0 ? 1 : (k < 4 ? 2 : 3); }
     __host__ __device__ static constexpr double post(int k) { return ((void)k, 1.0); }
-    __device__ static void stage(const double *in, double *o) { o[0] = in[0]; }
+    template <int PREC>
+    __host__ __device__ static void stage_p(const double *in, double *o) { o[0] = PREC == 0 ? 0.5 * in[0] : in[0]; }
+    template <bool M>
+    __device__ static void eval64(double *a, double dx, double dy, double dz, const double *f) {
+        const double w = twice_rsqrt_f64<M>(dx * dx + dy * dy + dz * dz);
+        const double w2 = w * w;
+        const double A = f[0] * w;
+        const double sv = A * w2;
+        a[0] += A;
+        a[1] += sv * dx;
+        a[2] += sv * dy;
+        a[3] += sv * dz;
+        a[4] += sv;
+        const double K = sv * w2;
+        const double kx = K * dx, ky = K * dy, kz = K * dz;
+        a[5] += kx * dx;
+        a[6] += ky * dy;
+        a[7] += kz * dz;
+        a[8] += kx * dy;
+        a[9] += kx * dz;
+        a[10] += ky * dz;
+    }
+    __device__ static void finish64(const double *a, double *o) {
+        o[0] = a[0];
+        for (int i = 0; i < 3; ++i)
+            o[1 + i] = -0.25 * a[1 + i];
+        const double d = 0.25 * a[4];
+        o[4] = 0.1875 * a[5] - d;
+        o[5] = 0.1875 * a[8];
+        o[6] = 0.1875 * a[9];
+        o[7] = 0.1875 * a[6] - d;
+        o[8] = 0.1875 * a[10];
+        o[9] = 0.1875 * a[7] - d;
+    }
     template <class R, bool M = true>
     __device__ static void eval(R *u, R dx, R dy, R dz, const R *f) {
+        if constexpr (sizeof(R) == 8) {
+            eval_by_acc64<UkLaplacePGradGrad>(u, dx, dy, dz, f);
+            return;
+        }
         R r2 = dx * dx + dy * dy + dz * dz;
         const auto rs = pair_rsqrt<M>(r2);
         R s = rs.s;
@@ -306,15 +366,62 @@ struct UkLaplacePGradGrad {
 //   grad grad p_ij = (15 c n_i n_j - 3 c delta_ij - 3 (n_i f_j + n_j f_i)) s^4
 // (the reference's r-polynomials over r^3, r^5, r^7 divided through by r^k; the literal 1/r^7
 // overflows FP32 below r ~ 3e-6, the unit-direction form only below r ~ 1e-9).
+// FP64 (c = f.r, w = 2/r): with v = c w^2 and e_j = (5/8) v r_j - f_j the Hessian is 3 w^5/32 (r_i e_j + r_j e_i) -
+// d_ij 3 c w^5/32; accumulators p (1/8), grad (1/8), r_i e_i w^5, (r_i e_j + r_j e_i) w^5, c w^5 (once).
 struct UkLaplaceDipolePGradGrad {
-    static constexpr int KS = 3, KS1 = 3, KL = 3, KT = 10;
+    static constexpr int KS = 3, KS1 = 3, KL = 3, KT = 10, ACC64 = 11;
     static constexpr bool UNMASKED_EVAL = true;
     static constexpr unsigned SRC_SCALE_MASK = 0x7u;
     __host__ __device__ static constexpr int deg(int k) { return k == 0 ? 1 : (k < 4 ? 2 : 3); }
     __host__ __device__ static constexpr double post(int k) { return ((void)k, 1.0); }
     __device__ static void stage(const double *in, double *o) { o[0] = in[0]; o[1] = in[1]; o[2] = in[2]; }
+    template <bool M>
+    __device__ static void eval64(double *a, double dx, double dy, double dz, const double *f) {
+        const double w = twice_rsqrt_f64<M>(dx * dx + dy * dy + dz * dz);
+        const double c = f[0] * dx + f[1] * dy + f[2] * dz;
+        const double w2 = w * w;
+        const double w3 = w2 * w;
+        const double w5 = w3 * w2;
+        const double v = c * w2;
+        const double m = v * w3;
+        const double mk = -0.75 * m;
+        a[0] += c * w3;
+        a[1] += f[0] * w3;
+        a[1] += dx * mk;
+        a[2] += f[1] * w3;
+        a[2] += dy * mk;
+        a[3] += f[2] * w3;
+        a[3] += dz * mk;
+        a[4] += m;
+        const double v5 = 0.625 * v;
+        const double ex = (v5 * dx - f[0]) * w5, ey = (v5 * dy - f[1]) * w5, ez = (v5 * dz - f[2]) * w5;
+        a[5] += dx * ex;
+        a[6] += dy * ey;
+        a[7] += dz * ez;
+        a[8] += dx * ey;
+        a[8] += dy * ex;
+        a[9] += dx * ez;
+        a[9] += dz * ex;
+        a[10] += dy * ez;
+        a[10] += dz * ey;
+    }
+    __device__ static void finish64(const double *a, double *o) {
+        for (int k = 0; k < 4; ++k)
+            o[k] = 0.125 * a[k];
+        const double d = 0.09375 * a[4];
+        o[4] = 0.1875 * a[5] - d;
+        o[5] = 0.09375 * a[8];
+        o[6] = 0.09375 * a[9];
+        o[7] = 0.1875 * a[6] - d;
+        o[8] = 0.09375 * a[10];
+        o[9] = 0.1875 * a[7] - d;
+    }
     template <class R, bool M = true>
     __device__ static void eval(R *u, R dx, R dy, R dz, const R *f) {
+        if constexpr (sizeof(R) == 8) {
+            eval_by_acc64<UkLaplaceDipolePGradGrad>(u, dx, dy, dz, f);
+            return;
+        }
         R r2 = dx * dx + dy * dy + dz * dz;
         const auto rs = pair_rsqrt<M>(r2);
         const R s = rs.s, s2 = rs.s2;
