@@ -679,13 +679,11 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         p->dn_src = rng_src_end[r0] - p->ds_begin;
         p->dlayout = direct_layout_uk(uk, precision, precision == STKFMM_PREC_FP64 ? direct_fp64_targets(p->KT) : T,
                                       p->dn_src, p->dn_trg, n_cu);
-        if (p->dlayout.chunks > 1) {
-            const hipError_t e = hipMalloc((void **)&p->d_partial,
-                                           sizeof(double) * p->dlayout.chunks * p->KT * (size_t)p->dn_trg);
-            if (e != hipSuccess) {
-                plan_free(p);
-                return hip_error(e, "plan workspace");
-            }
+        const hipError_t e = hipMalloc((void **)&p->d_partial,
+                                       sizeof(double) * p->dlayout.chunks * p->KT * (size_t)p->dn_trg);
+        if (e != hipSuccess) {
+            plan_free(p);
+            return hip_error(e, "plan workspace");
         }
         *plan_out = p;
         return STKFMM_OK;
@@ -747,10 +745,10 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
 
 static bool arr_ok(const stkfmm_array *a) { return a && a->ptr && a->stride >= 0 && a->fstride >= 0; }
 
-// one direct-sum launch over arrays that start at the first source and target
-static int enqueue_direct(int uk, int prec, const DirectLayout &l, int n_src, int n_trg, const DArr &sc, const DArr &v1,
-                          const DArr &v2, const DArr &tc, const OArr &out, const int *perm, double *partial,
-                          hipStream_t s) {
+// one direct-sum launch over arrays that start at the first source and target; partial holds l.chunks * KT *
+// n_trg doubles
+static DirectArgs direct_args(int uk, int n_src, int n_trg, const DArr &sc, const DArr &v1, const DArr &v2,
+                              const DArr &tc, const OArr &out, const int *perm, double *partial) {
     DirectArgs a{};
     a.sc = sc;
     a.v1 = v1;
@@ -762,8 +760,8 @@ static int enqueue_direct(int uk, int prec, const DirectLayout &l, int n_src, in
     a.scale = uker_scale(uk);
     a.n_src = n_src;
     a.n_trg = n_trg;
-    HIP_TRY(launch_direct(uk, prec, a, l, s), "direct sum launch");
-    return STKFMM_OK;
+    a.two_phase = direct_out_overlaps(a, uker_ks(uk), uker_ks1(uk), uker_kt(uk));
+    return a;
 }
 
 static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_array *sv, const stkfmm_array *sv2,
@@ -790,10 +788,9 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
             ++p->n_timed;
             HIP_TRY(hipEventRecord(ev[0], s), "event record");
         }
-        const int rc = enqueue_direct(p->uk, p->prec, p->dlayout, p->dn_src, p->dn_trg, from(a.sc, s0), from(a.v1, s0),
-                                      from(a.v2, s0), from(a.tc, t0), out, perm ? perm + t0 : nullptr, p->d_partial, s);
-        if (rc)
-            return rc;
+        const DirectArgs d = direct_args(p->uk, p->dn_src, p->dn_trg, from(a.sc, s0), from(a.v1, s0), from(a.v2, s0),
+                                         from(a.tc, t0), out, perm ? perm + t0 : nullptr, p->d_partial);
+        HIP_TRY(launch_direct(p->uk, p->prec, d, p->dlayout, s), "direct sum launch");
         if (timed) { // the partial sums of a chunked sum are added inside the first interval
             HIP_TRY(hipEventRecord(ev[1], s), "event record");
             HIP_TRY(hipEventRecord(ev[2], s), "event record");
@@ -1056,9 +1053,10 @@ int direct_plan(int uk, int prec, int n_src, int n_trg, stkfmm_plan **out) {
 // grow-only device buffers for the host-pointer entries
 struct Workspace {
     int device = -1;
-    // slot 0: host-pointer entries (inputs and output, packed); slot 1: adjoint partial sums
-    double *buf[2] = {nullptr, nullptr};
-    size_t cap[2] = {0, 0};
+    // slot 0: host-pointer entries (inputs and output, packed); slot 1: adjoint partial sums; slot 2: copies of
+    // wall-image inputs that the output overlaps
+    double *buf[3] = {nullptr, nullptr, nullptr};
+    size_t cap[3] = {0, 0, 0};
 };
 std::vector<Workspace> g_ws;
 
@@ -1101,8 +1099,13 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
         if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
             return rc;
         const DirectLayout l = direct_layout_uk(uk, prec, direct_targets_per_lane(prec, kt, n_trg), n_src, n_trg, n_cu);
-        return enqueue_direct(uk, prec, l, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
-                              DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, partial, s);
+        const DirectArgs a = direct_args(uk, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
+                                         DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, partial);
+        // (an output over an input, with more targets than the fixed array holds, goes on to a plan)
+        if (!a.two_phase || (long long)l.chunks * n_trg * kt <= 16 * kDirectPartialTargets) {
+            HIP_TRY(launch_direct(uk, prec, a, l, s), "direct sum launch");
+            return STKFMM_OK;
+        }
     }
     stkfmm_plan *p = nullptr;
     if ((rc = direct_plan(uk, prec, n_src, n_trg, &p)))
@@ -1223,17 +1226,34 @@ int wall_device(unsigned kernel, const double *sc, const double *sv, int n, cons
     if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
         return rc;
     const int ks = kernel == STKFMM_KERNEL_Stokes ? 3 : 4, kt = kernel == STKFMM_KERNEL_Stokes ? 3 : 6;
+    DirectArgs a{};
+    a.sc = DArr{sc, 3, 1};
+    a.v1 = a.v2 = DArr{sv, ks, 1};
+    a.tc = DArr{tc, 3, 1};
+    a.out = OArr{tv, kt, 1};
+    a.partial = partial;
+    a.scale = uker_scale(STKFMM_UKER_STOKES_VEL);
+    a.n_src = n;
+    a.n_trg = m;
+    if (direct_out_overlaps(a, ks, ks, kt)) {
+        // results over an input: the sums read a copy
+        const size_t N = (size_t)n, M = (size_t)m;
+        double *w = nullptr;
+        if ((rc = ws_get(2, (3 + ks) * N + 3 * M, &w)))
+            return rc;
+        HIP_TRY(hipMemcpyAsync(w, sc, sizeof(double) * 3 * N, hipMemcpyDeviceToDevice, s), "copy inputs");
+        HIP_TRY(hipMemcpyAsync(w + 3 * N, sv, sizeof(double) * ks * N, hipMemcpyDeviceToDevice, s), "copy inputs");
+        HIP_TRY(hipMemcpyAsync(w + (3 + ks) * N, tc, sizeof(double) * 3 * M, hipMemcpyDeviceToDevice, s), "copy inputs");
+        a.sc.p = w;
+        a.v1.p = a.v2.p = w + 3 * N;
+        a.tc.p = w + (3 + ks) * N;
+    }
     // target slabs keep the launch inside its index range
     const int slab = 1 << 29;
+    const double *t_first = a.tc.p;
     for (long long t0 = 0; t0 < m; t0 += slab) {
-        DirectArgs a{};
-        a.sc = DArr{sc, 3, 1};
-        a.v1 = a.v2 = DArr{sv, ks, 1};
-        a.tc = DArr{tc + 3 * t0, 3, 1};
-        a.out = OArr{tv + kt * t0, kt, 1};
-        a.partial = partial;
-        a.scale = uker_scale(STKFMM_UKER_STOKES_VEL);
-        a.n_src = n;
+        a.tc.p = t_first + 3 * t0;
+        a.out.p = tv + kt * t0;
         a.n_trg = (int)std::min<long long>(slab, m - t0);
         HIP_TRY(launch_wall(kernel == STKFMM_KERNEL_RPY, a, n_cu, s), "wall images launch");
     }

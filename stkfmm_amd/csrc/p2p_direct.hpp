@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
             for (int w = 0; w < W; ++w)
                 v += smem[(w * KG + q) * TT + i];
             v *= post_for<K, PREC>(k);
-            if (gridDim.y == 1) {
+            if (!a.two_phase) {
                 const long long o = a.perm ? (long long)a.perm[tb + i] : tb + i;
                 a.out.p[o * a.out.s + k * a.out.fs] += a.scale * v;
             } else {

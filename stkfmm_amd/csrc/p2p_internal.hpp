@@ -94,7 +94,8 @@ struct DirectArgs {
     DArr sc, v1, v2, tc; // as ItemArgs
     OArr out;
     const int *perm;     // output row of target i (null: identity)
-    double *partial;     // [chunk][KT][n_trg], used when there are several chunks
+    double *partial;     // [chunk][KT][n_trg], used when there are several chunks, and when out overlaps an input
+    int two_phase;       // the sums go to partial first
     double scale;        // ScaleFactor of the kernel
     int n_src, n_trg;
     int ls, unit, tail_begin, tail_ls, chunk_tiles; // DirectLayout
@@ -270,6 +271,9 @@ int uker_run(int uk);
 // device memory for the chunks' partial sums of the direct-sum entries on the current device
 // (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
 int direct_partial_ptr(double **out);
+// out shares memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
+// the item and reduce kernels do
+bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt);
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s);
 hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s);
 // equivalent / check surfaces (surface.hip)

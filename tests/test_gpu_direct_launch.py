@@ -106,3 +106,28 @@ def test_one_launch_nonfinite_and_overflow(prec):
         if what == "close":
             ref = O.direct(int(uk), src, val, trg[3:4])
             assert np.abs(got[0][3] - ref[0]).max() <= (1e-12 if prec == 0 else 1e-6) * np.abs(ref[0]).max()
+
+
+def test_output_over_an_input():
+    """f += K f: everything is read before anything is written, in every direct entry."""
+    n = 700  # one source chunk
+    rng = np.random.default_rng(8)
+    x, f = rng.random((n, 3)), rng.normal(size=(n, 3))
+    ref = f + O.direct(int(S.UKER.STOKES_VEL), x, f, x)
+    d_x = to_dev(x)
+    plan = S.Plan(S.UKER.STOKES_VEL, 0, n, n, [0], [n], None, [0, 1], [0], [n])
+    for name, call in (("entry", lambda v: S.p2p_device(S.KERNEL.Stokes, S.PPKERNEL.SLS2T, d_x, v, d_x, v)),
+                       ("no-alloc", lambda v: S.p2p_device(S.KERNEL.Stokes, S.PPKERNEL.SLS2T, d_x, v, d_x, v,
+                                                           no_alloc=True)),
+                       ("plan", lambda v: plan.execute(d_x, v, d_x, v))):
+        say(f"direct in place {name}")
+        d_f = to_dev(f)
+        call(d_f)
+        l2, mx = O.max_error(host(d_f), ref)
+        assert l2 < FP64_TOL and mx < FP64_TOL, (name, l2, mx)
+    z = x.copy()
+    z[:, 2] *= 0.5
+    d_z, d_f = to_dev(z), to_dev(f)
+    S.wall_device(S.KERNEL.Stokes, d_z, d_f, d_z, d_f)
+    l2, mx = O.max_error(host(d_f), f + O.wall(int(S.KERNEL.Stokes), z, f, z))
+    assert l2 < FP64_TOL and mx < FP64_TOL, ("wall", l2, mx)
