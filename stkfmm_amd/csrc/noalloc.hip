@@ -259,6 +259,7 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
     a.n_queues = 1;
     a.partial = (double *)(base + L.partial);
     a.n_src_rec = nSrc;
+    a.whole_out = 0;
     const int grid = (int)(n_items < (long long)n_cu * bpc ? n_items : (long long)n_cu * bpc);
     if ((e = launch_items(uk, precision, T, grid, a, s)) != hipSuccess)
         return fail(STKFMM_ERR_HIP, "no-alloc direct sum: item kernel launch failed");

@@ -248,6 +248,7 @@ struct stkfmm_plan {
     int uk = 0, prec = 0, T = 2, TT = 128, KS = 0, KS1 = 0, KT = 0;
     int n_src = 0, n_trg = 0;
     int n_items = 0, n_tiles = 0, n_ranges = 0;
+    int n_split_tiles = 0; // the first tiles: those of several items
     int grid = 0, persistent = 1;
     long long pairs = 0;
     int device = 0;
@@ -563,6 +564,8 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
                 item_group.push_back(g);
             }
             tl.slot_end = (int)items.size();
+            if (tl.slot_end - tl.slot_begin == 1)
+                items.back().lsplit |= kItemWhole;
             tiles.push_back(tl);
         }
         if ((int)items.size() > group_items.back())
@@ -689,6 +692,10 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         return STKFMM_OK;
     }
 
+    // the tiles that always need the reduction first
+    p->n_split_tiles = (int)(std::stable_partition(tiles.begin(), tiles.end(),
+                                                   [](const Tile &t) { return t.slot_end - t.slot_begin != 1; }) -
+                             tiles.begin());
     int r;
     if ((r = upload(&p->d_items, items, "plan items")) || (r = upload(&p->d_ranges, ranges, "plan ranges")) ||
         (r = upload(&p->d_tiles, tiles, "plan tiles")) || (r = upload(&p->d_qptr, q_ptr, "plan queues"))) {
@@ -762,6 +769,19 @@ static DirectArgs direct_args(int uk, int n_src, int n_trg, const DArr &sc, cons
     a.n_trg = n_trg;
     a.two_phase = direct_out_overlaps(a, uker_ks(uk), uker_ks1(uk), uker_kt(uk));
     return a;
+}
+
+// a plan's output rows share memory with its inputs (direct_out_overlaps)
+static bool out_overlaps(const stkfmm_plan *p, const ItemArgs &a) {
+    DirectArgs d{};
+    d.sc = a.sc;
+    d.v1 = a.v1;
+    d.v2 = a.v2;
+    d.tc = a.tc;
+    d.out = a.out;
+    d.n_src = p->n_src;
+    d.n_trg = p->n_trg;
+    return direct_out_overlaps(d, p->KS, p->KS1, p->KT);
 }
 
 static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_array *sv, const stkfmm_array *sv2,
@@ -840,15 +860,21 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
     a.n_queues = p->n_queues;
     a.partial = p->d_partial;
     a.n_src_rec = p->n_src;
+    a.out = OArr{tv->ptr, tv->stride, tv->fstride};
+    a.perm = perm;
+    a.scale = uker_scale(p->uk);
+    // whole tiles go straight to the output, unless it shares memory with an input (ordered points are the
+    // plan's own copies)
+    a.whole_out = p->sorted || !out_overlaps(p, a);
     ReduceArgs ra;
     ra.tiles = p->d_tiles;
-    ra.n_tiles = p->n_tiles;
+    ra.n_tiles = a.whole_out ? p->n_split_tiles : p->n_tiles;
     ra.kt = p->KT;
     ra.tt = p->TT;
     ra.partial = p->d_partial;
-    ra.out = OArr{tv->ptr, tv->stride, tv->fstride};
+    ra.out = a.out;
     ra.perm = perm;
-    ra.scale = uker_scale(p->uk);
+    ra.scale = a.scale;
     const bool timed = allow_timing && p->timing;
     hipEvent_t *ev = timed ? &p->ev[3 * (p->n_timed % stkfmm_plan::kRing)] : nullptr;
     if (timed) {
@@ -879,7 +905,7 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
     if (timed)
         HIP_TRY(hipEventRecord(ev[1], s), "event record");
     // permuted rows with many tiles: one contiguous write per target (same sums, same order)
-    if (perm && p->n_tiles >= 1024)
+    if (perm && ra.n_tiles >= 1024)
         HIP_TRY(launch_reduce_rows(ra, s), "p2p reduce launch");
     else
         HIP_TRY(launch_reduce(ra, s), "p2p reduce launch");

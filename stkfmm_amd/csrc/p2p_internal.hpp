@@ -31,8 +31,11 @@ struct Item {
     int cost;       // sources in the item (scheduling key)
     int lsplit;     // log2 of the lanes per target: a tile of n targets uses 2^lsplit lanes per
                     // target when n * 2^lsplit <= 64*T; each of those lanes takes every
-                    // 2^lsplit-th staged source and the partial sums meet by wavefront shuffles
+                    // 2^lsplit-th staged source and the partial sums meet by wavefront shuffles;
+                    // plus kItemWhole when the item is its tile's only one
 };
+// an item that holds its tile's whole source list: it may add its sums to the output itself
+constexpr int kItemWhole = 256;
 
 // a target tile and the partial-sum slots that cover it
 struct Tile {
@@ -68,6 +71,12 @@ struct ItemArgs {
     int n_queues;
     double *partial;      // [slot][KT][64*T]
     long long n_src_rec;  // scalar-broadcast variant: sources per staged record copy
+    // output, for the items marked kItemWhole when whole_out is set (else they write their partial slot
+    // like the others); perm and scale as in ReduceArgs
+    OArr out;
+    const int *perm;
+    double scale;
+    int whole_out;
 };
 
 // scalar-broadcast variant: per-source records staged once per execute (one copy per level)

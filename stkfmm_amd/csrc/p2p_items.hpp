@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(kWave) STKP2P_ITEM_ATTR
 __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_kernel(ItemArgs a) {
     using K = typename UkerOf<UK>::type;
     constexpr int KL = StagedCount<K, PREC>::value, KT = K::KT, KS = K::KS, KS1 = K::KS1;
-    constexpr int TT = kWave * T, NA = AccCount<K, PREC>::value;
+    constexpr int NA = AccCount<K, PREC>::value;
 
     // FP64: values as [KL][tile] (two consecutive sources per 16-byte read);
     // mixed: FP32 values as 16-byte aligned rows [tile][KLP] (one source per few 16-byte reads,
@@ -160,7 +160,7 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
         const Item item = a.items[it];
         const double lam = (PREC == 0) ? 1.0 : ldexp(1.0, item.level);
         // lanes per target (uniform): lane = target slot * split + sub
-        const int ls = item.lsplit;
+        const int ls = item.lsplit & (kItemWhole - 1);
         const int split = 1 << ls;
         const int sub = lane & (split - 1);
         const int slot0 = lane >> ls;
@@ -478,17 +478,7 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
 #pragma unroll
         for (int t = 0; t < T; ++t)
             finish_acc<K, PREC>(acc[t], out[t]);
-        double *dst = a.partial + (long long)item.slot * KT * TT;
-#pragma unroll
-        for (int k = 0; k < KT; ++k) {
-            const double osc = ((PREC == 0) ? 1.0 : ldexp(1.0, K::deg(k) * item.level)) * post_for<K, PREC>(k);
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const int i = slot0 + tstride * t;
-                if (sub == 0 && i < item.trg_count)
-                    dst[(long long)k * TT + i] = out[t][k] * osc;
-            }
-        }
+        write_sums<K, PREC, T>(item, out, slot0, tstride, sub == 0);
     }
 }
 

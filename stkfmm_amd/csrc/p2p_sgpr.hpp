@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
     using K = typename UkerOf<UK>::type;
     using L = RecLayout<K, PREC>;
     constexpr int KL = L::KL, KT = K::KT;
-    constexpr int TT = kWave * T, NA = AccCount<K, PREC>::value;
+    constexpr int NA = AccCount<K, PREC>::value;
     const int lane = threadIdx.x;
     ItemCursor cur(a);
     for (;;) {
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
 
         const Item item = a.items[it];
         const double lam = (PREC == 0) ? 1.0 : ldexp(1.0, item.level);
-        const int ls = item.lsplit;
+        const int ls = item.lsplit & (kItemWhole - 1);
         const int split = 1 << ls;
         const int sub = lane & (split - 1);
         const int slot0 = lane >> ls;
@@ -245,17 +245,7 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
 #pragma unroll
         for (int t = 0; t < T; ++t)
             finish_acc<K, PREC>(acc[t], out[t]);
-        double *dst = a.partial + (long long)item.slot * KT * TT;
-#pragma unroll
-        for (int k = 0; k < KT; ++k) {
-            const double osc = ((PREC == 0) ? 1.0 : ldexp(1.0, K::deg(k) * item.level)) * post_for<K, PREC>(k);
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const int i = slot0 + tstride * t;
-                if (sub == 0 && i < item.trg_count)
-                    dst[(long long)k * TT + i] = out[t][k] * osc;
-            }
-        }
+        write_sums<K, PREC, T>(item, out, slot0, tstride, sub == 0);
     }
 }
 
