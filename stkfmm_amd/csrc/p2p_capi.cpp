@@ -366,6 +366,11 @@ static bool direct_sorts_points(int n_src, int n_trg) {
     return (n_src >= kDirectSortMin && n_trg >= kDirectSortMin) || !direct_sizes(n_src, n_trg);
 }
 
+// direct sums that are one launch
+static bool direct_in_one_call(int uk, int prec, int n_src, int n_trg) {
+    return !direct_sorts_points(n_src, n_trg) && direct_in_one_launch(prec, uk);
+}
+
 extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision, int n_src, int n_trg,
                                   int n_groups, const int *grp_trg_begin, const int *grp_trg_end,
                                   const int *grp_level, const int *grp_rng_ptr, const int *rng_src_begin,
@@ -672,8 +677,7 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     // 4.0 against 4.3 ms).  The item list above stays for stkfmm_plan_stats.
     const stkfmm_tune no_tune{};
     if (n_groups == 1 && !grp_level && std::memcmp(&tn, &no_tune, sizeof(tn)) == 0 && p->n_items > 0 &&
-        grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && !direct_sorts_points(n_src, n_trg) &&
-        direct_in_one_launch(precision, uk)) {
+        grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && direct_in_one_call(uk, precision, n_src, n_trg)) {
         const int r0 = grp_rng_ptr[0];
         p->direct = true;
         p->dt_begin = grp_trg_begin[0];
@@ -1109,8 +1113,9 @@ int ws_get(int slot, size_t n, double **out) {
     return STKFMM_OK;
 }
 
+// the device-pointer entries' sum; store (only where direct_in_one_call): tv = sum instead of tv += sum
 int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *sv, int n_trg, const double *tc,
-                   double *tv, hipStream_t s) {
+                   double *tv, hipStream_t s, bool store = false) {
     if (n_src < 0 || n_trg < 0)
         return set_error(STKFMM_ERR_ARG, "negative point count");
     if (n_src == 0 || n_trg == 0)
@@ -1119,14 +1124,15 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
     const int ks = uker_ks(uk), ks1 = uker_ks1(uk), kt = uker_kt(uk);
     int rc;
-    if (!direct_sorts_points(n_src, n_trg) && direct_in_one_launch(prec, uk)) {
+    if (direct_in_one_call(uk, prec, n_src, n_trg)) {
         int n_cu = 0;
         double *partial = nullptr;
         if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
             return rc;
         const DirectLayout l = direct_layout_uk(uk, prec, direct_targets_per_lane(prec, kt, n_trg), n_src, n_trg, n_cu);
-        const DirectArgs a = direct_args(uk, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
+        DirectArgs a = direct_args(uk, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
                                          DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, partial);
+        a.store = store;
         // (an output over an input, with more targets than the fixed array holds, goes on to a plan)
         if (!a.two_phase || (long long)l.chunks * n_trg * kt <= 16 * kDirectPartialTargets) {
             HIP_TRY(launch_direct(uk, prec, a, l, s), "direct sum launch");
@@ -1161,13 +1167,21 @@ int pinned_get(size_t n, double **out) {
     return STKFMM_OK;
 }
 
-// A host-pointer evaluation: the three inputs are packed into the pinned buffer and moved in one
-// copy; the device output starts at zero and comes back in one copy, after one synchronisation;
-// the caller's trgValue += result is then done here (the same additions as on the device, since
-// 0 + x is exact).  eval(d_sc, d_sv, d_tc, d_tv) enqueues the device work on the null stream.
+// Up to this size the kernels move a host-pointer call's data themselves: one copy kernel reads the
+// inputs from the pinned buffer, and the sums are stored into it.  Above, the copy engines do.
+constexpr size_t kKernelCopyBytes = size_t(1) << 20;
+
+// A host-pointer evaluation: the three inputs are packed into the pinned buffer and moved to the device; the
+// result comes back through the pinned buffer, after one synchronisation; the caller's trgValue += result
+// is then done here (the same additions as on the device, since 0 + x is exact).  eval(d_sc, d_sv, d_tc,
+// d_tv) enqueues the device work on the null stream; with `stores` it overwrites d_tv (which may be host
+// memory), else it adds to it.
+// With engine copies each way and a cleared output 1,000 x 1,000 LapPGrad through evaluateKernel took 46 us,
+// so 33 (of them 16 us from the launches to the end of the synchronisation, 12 us of GPU time); 24 Ker_t
+// blocks 1.19 -> 0.94 ms.
 template <class Eval>
 int host_roundtrip(size_t ks, size_t kt, int n_src, const double *sc, const double *sv, int n_trg,
-                   const double *tc, double *tv, Eval eval) {
+                   const double *tc, double *tv, bool stores, Eval eval) {
     const size_t n_sc = 3 * (size_t)n_src, n_sv = ks * n_src, n_tc = 3 * (size_t)n_trg, n_tv = kt * n_trg;
     const size_t n_in = n_sc + n_sv + n_tc;
     double *h = nullptr, *d = nullptr;
@@ -1177,15 +1191,22 @@ int host_roundtrip(size_t ks, size_t kt, int n_src, const double *sc, const doub
     std::memcpy(h, sc, sizeof(double) * n_sc);
     std::memcpy(h + n_sc, sv, sizeof(double) * n_sv);
     std::memcpy(h + n_sc + n_sv, tc, sizeof(double) * n_tc);
-    double *d_tv = d + n_in, *h_tv = h + n_in;
-    HIP_TRY(hipMemcpyAsync(d, h, sizeof(double) * n_in, hipMemcpyHostToDevice, nullptr), "copy inputs");
-    HIP_TRY(hipMemsetAsync(d_tv, 0, sizeof(double) * n_tv, nullptr), "clear output");
+    double *const h_tv = h + n_in;
+    const bool to_host = stores && sizeof(double) * n_tv <= kKernelCopyBytes;
+    double *const d_tv = to_host ? h_tv : d + n_in;
+    if (sizeof(double) * n_in <= kKernelCopyBytes)
+        HIP_TRY(launch_copy(h, d, n_in, nullptr), "copy inputs");
+    else
+        HIP_TRY(hipMemcpyAsync(d, h, sizeof(double) * n_in, hipMemcpyHostToDevice, nullptr), "copy inputs");
+    if (!stores)
+        HIP_TRY(hipMemsetAsync(d_tv, 0, sizeof(double) * n_tv, nullptr), "clear output");
     rc = eval(d, d + n_sc, d + n_sc + n_sv, d_tv);
     if (rc) {
         (void)hipStreamSynchronize(nullptr);
         return rc;
     }
-    HIP_TRY(hipMemcpyAsync(h_tv, d_tv, sizeof(double) * n_tv, hipMemcpyDeviceToHost, nullptr), "copy result");
+    if (!to_host)
+        HIP_TRY(hipMemcpyAsync(h_tv, d_tv, sizeof(double) * n_tv, hipMemcpyDeviceToHost, nullptr), "copy result");
     HIP_TRY(hipStreamSynchronize(nullptr), "synchronise");
     for (size_t i = 0; i < n_tv; ++i)
         tv[i] += h_tv[i];
@@ -1200,9 +1221,10 @@ int eval_host_uk(int uk, int prec, int n_src, const double *sc, const double *sv
         return STKFMM_OK;
     if (!sc || !sv || !tc || !tv)
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
-    return host_roundtrip(uker_ks(uk), uker_kt(uk), n_src, sc, sv, n_trg, tc, tv,
+    const bool stores = direct_in_one_call(uk, prec, n_src, n_trg);
+    return host_roundtrip(uker_ks(uk), uker_kt(uk), n_src, sc, sv, n_trg, tc, tv, stores,
                           [&](const double *d_sc, const double *d_sv, const double *d_tc, double *d_tv) {
-                              return eval_device_uk(uk, prec, n_src, d_sc, d_sv, n_trg, d_tc, d_tv, nullptr);
+                              return eval_device_uk(uk, prec, n_src, d_sc, d_sv, n_trg, d_tc, d_tv, nullptr, stores);
                           });
 }
 
@@ -1246,7 +1268,7 @@ extern "C" int stkfmm_p2p_eval_device(unsigned kernel, unsigned p2p, int precisi
 namespace {
 // one direct sum of source-and-image pairs (wall.hip)
 int wall_device(unsigned kernel, const double *sc, const double *sv, int n, const double *tc, double *tv, int m,
-                hipStream_t s) {
+                hipStream_t s, bool store = false) {
     int n_cu = 0, rc;
     double *partial = nullptr;
     if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
@@ -1258,6 +1280,7 @@ int wall_device(unsigned kernel, const double *sc, const double *sv, int n, cons
     a.tc = DArr{tc, 3, 1};
     a.out = OArr{tv, kt, 1};
     a.partial = partial;
+    a.store = store;
     a.scale = uker_scale(STKFMM_UKER_STOKES_VEL);
     a.n_src = n;
     a.n_trg = m;
@@ -1329,9 +1352,9 @@ extern "C" int stkfmm_wall_evaluate(unsigned kernel, int precision, int nSL, con
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
     const size_t ks = kernel == STKFMM_KERNEL_Stokes ? 3 : 4, kt = kernel == STKFMM_KERNEL_Stokes ? 3 : 6;
     std::lock_guard<std::mutex> lk(g_mu);
-    return host_roundtrip(ks, kt, nSL, srcCoord, srcValue, nTrg, trgCoord, trgValue,
+    return host_roundtrip(ks, kt, nSL, srcCoord, srcValue, nTrg, trgCoord, trgValue, true,
                           [&](const double *d_sc, const double *d_sv, const double *d_tc, double *d_tv) {
-                              return wall_device(kernel, d_sc, d_sv, nSL, d_tc, d_tv, nTrg, nullptr);
+                              return wall_device(kernel, d_sc, d_sv, nSL, d_tc, d_tv, nTrg, nullptr, true);
                           });
 }
 

@@ -305,8 +305,11 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
         }
         __syncthreads();
         const int nk = (KT - k0 < KG) ? KT - k0 : KG;
+        // consecutive threads write consecutive doubles: of the (usually contiguous) output rows, or of a
+        // component's partial sums
         for (int e = threadIdx.x; e < nk << lgu; e += blockDim.x) {
-            const int q = e >> lgu, i = e & ((1 << lgu) - 1), k = k0 + q;
+            const int i = a.two_phase ? e & ((1 << lgu) - 1) : e / nk;
+            const int q = a.two_phase ? e >> lgu : e - nk * i, k = k0 + q;
             if (tb + i >= te)
                 continue;
             double v = 0.0;
@@ -315,7 +318,8 @@ __global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectA
             v *= post_for<K, PREC>(k);
             if (!a.two_phase) {
                 const long long o = a.perm ? (long long)a.perm[tb + i] : tb + i;
-                a.out.p[o * a.out.s + k * a.out.fs] += a.scale * v;
+                double *const p = a.out.p + o * a.out.s + k * a.out.fs;
+                *p = a.store ? a.scale * v : *p + a.scale * v;
             } else {
                 a.partial[((long long)blockIdx.y * KT + k) * a.n_trg + tb + i] = v;
             }

@@ -105,6 +105,7 @@ struct DirectArgs {
     const int *perm;     // output row of target i (null: identity)
     double *partial;     // [chunk][KT][n_trg], used when there are several chunks, and when out overlaps an input
     int two_phase;       // the sums go to partial first
+    int store;           // out = scale * sum (else out += scale * sum)
     double scale;        // ScaleFactor of the kernel
     int n_src, n_trg;
     int ls, unit, tail_begin, tail_ls, chunk_tiles; // DirectLayout
@@ -283,6 +284,8 @@ int direct_partial_ptr(double **out);
 // out shares memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
 // the item and reduce kernels do
 bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt);
+// dst[0, n) = src[0, n) by a kernel (small host-to-device copies)
+hipError_t launch_copy(const double *src, double *dst, size_t n, hipStream_t s);
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s);
 hipError_t launch_direct(int uk, int prec, DirectArgs a, const DirectLayout &l, hipStream_t s);
 // equivalent / check surfaces (surface.hip)

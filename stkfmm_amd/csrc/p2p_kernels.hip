@@ -163,17 +163,36 @@ hipError_t launch_stage_records(int uk, int prec, const StageArgs &a, int n_copi
     return o ? o->stage(prec, a, n_copies, s) : hipErrorInvalidValue;
 }
 
-// out(perm[i], k) += scale * sum over the chunks, in chunk order, of partial[chunk][k][i]
+// out(perm[i], k) += scale * sum over the chunks, in chunk order, of partial[chunk][k][i] (or = with a.store);
+// a workgroup takes 64 targets, its threads consecutive doubles of their output rows
 __global__ void __launch_bounds__(256) direct_reduce_kernel(DirectArgs a, int chunks, int kt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-    if (i >= a.n_trg)
-        return;
-    double s = 0.0;
+    const int i0 = (int)blockIdx.x * 64, n = min(64, a.n_trg - i0) * kt;
+    for (int e = threadIdx.x; e < n; e += 256) {
+        const int r = (unsigned)e / (unsigned)kt, k = e - r * kt;
+        const long long i = i0 + r;
+        double s = 0.0;
 #pragma unroll 8
-    for (int c = 0; c < chunks; ++c)
-        s += a.partial[((long long)c * kt + k) * a.n_trg + i];
-    const long long o = a.perm ? (long long)a.perm[i] : i;
-    a.out.p[o * a.out.s + k * a.out.fs] += a.scale * s;
+        for (int c = 0; c < chunks; ++c)
+            s += a.partial[((long long)c * kt + k) * a.n_trg + i];
+        const long long o = a.perm ? (long long)a.perm[i] : i;
+        double *const p = a.out.p + o * a.out.s + k * a.out.fs;
+        *p = a.store ? a.scale * s : *p + a.scale * s;
+    }
+}
+
+__global__ void __launch_bounds__(256) copy_kernel(const double *src, double *dst, size_t n) {
+    const size_t step = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
+        dst[i] = src[i];
+}
+
+hipError_t launch_copy(const double *src, double *dst, size_t n, hipStream_t s) {
+    if (n == 0)
+        return hipSuccess;
+    // one double per thread up to 512 workgroups
+    const size_t blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(copy_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, s, src, dst, n);
+    return hipGetLastError();
 }
 
 int uker_run(int uk) {
@@ -203,8 +222,7 @@ bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt) {
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s) {
     if (!a.two_phase)
         return hipSuccess;
-    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 255) / 256), (unsigned)kt), dim3(256), 0, s, a,
-                       chunks, kt);
+    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 63) / 64)), dim3(256), 0, s, a, chunks, kt);
     return hipGetLastError();
 }
 

@@ -51,7 +51,7 @@ __device__ inline int next_item(const ItemArgs &a, ItemCursor &c, int lane) {
 // tile's only one, straight into the output with the reduction's own operations (out += scale * sum) --
 // no partial sums to write and read again, and no reduction where every tile is such.  Surface lists (one
 // leaf's points against its surface) are all such tiles: the four PVel lists of a 262,144-point tree, mixed,
-// 1.65 -> 1.58 ms; smaller sums 0.55 -> 0.45 ms
+// 1.65 -> 1.58 ms.
 template <class K, int PREC, int T>
 __device__ __forceinline__ void write_sums(const Item &item, const double (&out)[T][K::KT], int slot0, int tstride,
                                            bool mine) {
