@@ -1448,6 +1448,14 @@ extern "C" int stkfmm_p2p_vjp_device(int uker, int precision, int nSrc, const do
             l.T = 4;
         }
     }
+    // FP64: fewer targets per lane while the waves (one target tile x one source tile at the least) would not
+    // fill the SIMDs twice: 3,001 x 2,503 PVel 36.1 -> 30.5 us, 1,000 x 9,000 48.1 -> 42.4 us, with one
+    // reduction launch instead of three in both.  (Mixed mode's FP32 sums follow the tiles, so it keeps them.)
+    if (precision == STKFMM_PREC_FP64) {
+        const long long st = (nSrc + kSrcTile - 1) / kSrcTile;
+        while (l.T > 1 && (nTrg + kWave * l.T - 1LL) / (kWave * l.T) * st < 8LL * n_cu)
+            l.T /= 2;
+    }
     if (const char *e = std::getenv("STKFMM_VJP_T")) { // tuning and tests: 1, 2, 4, or 8 (mixed)
         const long t = std::strtol(e, nullptr, 10);
         const bool t4 = t == 4 && (precision == STKFMM_PREC_MIXED || vjp_fp64_four_targets(uker));

@@ -11,6 +11,7 @@
 //   The launch entries below dispatch through the per-micro-kernel UkerOps table.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "p2p_internal.hpp"
@@ -301,7 +302,7 @@ double uker_scale(int uk) {
 template <int UK, int PREC, int T>
 static hipError_t launch_vjp_t(const VjpArgs &a, const VjpLayout &l, double *partial, hipStream_t s) {
     using V = typename VjpOf<UK>::type;
-    constexpr int KS = V::KS, ND = 3 + KS;
+    constexpr int KS = V::KS;
     if (a.n_trg == 0 || a.n_src == 0) {
         if (a.g_tc)
             zero_fill(a.g_tc, 3LL * a.n_trg, s);
@@ -317,16 +318,9 @@ static hipError_t launch_vjp_t(const VjpArgs &a, const VjpLayout &l, double *par
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    const unsigned bt = (unsigned)((a.n_trg + 255) / 256), bs = (unsigned)((a.n_src + 255) / 256);
-    if (a.g_tc)
-        hipLaunchKernelGGL(vjp_reduce_kernel, dim3(bt, 3), dim3(256), 0, s, (const double *)tpart, a.n_trg, 3,
-                           l.n_chunks, 0, 3, a.g_tc, 3, 0, a.scale);
-    if (a.g_sc)
-        hipLaunchKernelGGL(vjp_reduce_kernel, dim3(bs, 3), dim3(256), 0, s, (const double *)spart, a.n_src, ND,
-                           l.n_blocks, 0, 3, a.g_sc, 3, 0, a.scale);
-    if (a.g_sv)
-        hipLaunchKernelGGL(vjp_reduce_kernel, dim3(bs, ND - 3), dim3(256), 0, s, (const double *)spart, a.n_src, ND,
-                           l.n_blocks, 3, ND, a.g_sv, KS, 0, a.scale);
+    const VjpReduce r{tpart, spart, a.g_tc, a.g_sc, a.g_sv, a.n_src, a.n_trg, l.n_chunks, l.n_blocks, KS, a.scale};
+    const unsigned n = (unsigned)std::max(a.n_src, a.n_trg);
+    hipLaunchKernelGGL(vjp_reduce_kernel, dim3((n + 255) / 256, 6 + KS), dim3(256), 0, s, r);
     return hipGetLastError();
 }
 

@@ -116,13 +116,36 @@ vjp_pair_kernel(VjpPass a) {
 #pragma unroll
             for (int d = 0; d < ND; ++d)
                 rs[d] = CT(0);
+            // Few targets per lane: such passes run one or two waves per SIMD, which leave the step's latency
+            // exposed.  The next step's source is read from LDS while this one is evaluated, and two steps
+            // are unrolled (3,001 x 2,503 Stokeslet, kernel and reduction, 30.3 -> 28.3 -> 26.7 us mixed; not
+            // for the nine- and 13-value sources, which spill: fused PVel 30,000^2 FP64 3.88 -> 4.53 ms, and
+            // mixed PVel and RPY, 20,000 x 3,000, 120 -> 124 us, are not unrolled).
+            constexpr bool AHEAD = T <= 2 && KS <= 4;
+            constexpr int STEPS = AHEAD && (PREC == 0 || KS <= 3) ? 2 : 1;
+            double px, py, pz;
+            CT pf[KS];
+            auto read = [&](int j) {
+                px = s_x[j];
+                py = s_y[j];
+                pz = s_z[j];
+#pragma unroll
+                for (int q = 0; q < KS; ++q)
+                    pf[q] = s_v[q][j];
+            };
+            if constexpr (AHEAD)
+                read(lane);
+#pragma unroll STEPS
             for (int k = 0; k < kSrcTile; ++k) {
-                const int j = (lane + k) & (kSrcTile - 1);
-                const double sx = s_x[j], sy = s_y[j], sz = s_z[j];
+                if constexpr (!AHEAD)
+                    read((lane + k) & (kSrcTile - 1));
+                const double sx = px, sy = py, sz = pz;
                 CT f[KS];
 #pragma unroll
                 for (int q = 0; q < KS; ++q)
-                    f[q] = s_v[q][j];
+                    f[q] = pf[q];
+                if constexpr (AHEAD)
+                    read((lane + k + 1) & (kSrcTile - 1));
                 // mixed mode: this step's source-value terms over the lane's T targets are summed
                 // apart and added to the rotating FP32 sums once, so those take 64 additions per target
                 // tile whatever T is.  Added straight in (2 FMAs per component per target), the value
@@ -178,21 +201,33 @@ vjp_pair_kernel(VjpPass a) {
     }
 }
 
-// out[i*ld + off + d] = scale * sum_c partial[c][d][i] for d = d0 + blockIdx.y (grid.y = d1 - d0:
-// one block row per component, so small point counts still give enough blocks); chunks are summed
-// in chunk order, so the result does not depend on the grid shape
-__global__ void vjp_reduce_kernel(const double *partial, int n, int nd, int nchunk, int d0, int d1,
-                                  double *out, int ld, int off, double scale) {
+// The partial sums of all outputs in one launch: blockIdx.y is a component of the target position gradient
+// (0-2), the source position gradient (3-5) or the source value gradient (6 ..), one block row each so that
+// small point counts still give enough blocks; out[i*ld + d] = scale * sum_c partial[c][d][i], chunks (or
+// blocks) in order, so the result does not depend on the grid shape.  (Three launches before: 3,001 x 2,503
+// Stokeslet adjoint 35.3 -> 30.3 us, 500 x 600 20.2 -> 15.4 us mixed.)
+struct VjpReduce {
+    const double *tpart, *spart;
+    double *g_tc, *g_sc, *g_sv; // null: not asked for
+    int n_src, n_trg, n_chunks, n_blocks, ks;
+    double scale;
+};
+__global__ void __launch_bounds__(256) vjp_reduce_kernel(VjpReduce a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int d = d0 + (int)blockIdx.y;
-    if (i >= n || out == nullptr || d >= d1)
+    const int c = blockIdx.y;
+    const bool trg = c < 3, pos = c < 6;
+    double *const out = trg ? a.g_tc : (pos ? a.g_sc : a.g_sv);
+    const int n = trg ? a.n_trg : a.n_src, nd = trg ? 3 : 3 + a.ks, d = trg ? c : c - 3;
+    if (i >= n || out == nullptr)
         return;
+    const double *const partial = (trg ? a.tpart : a.spart) + (long long)d * n + i;
+    const int m = trg ? a.n_chunks : a.n_blocks;
     double s = 0.0;
     // unrolled so that the loads of several chunks are in flight together (the adds keep chunk order)
 #pragma unroll 8
-    for (int c = 0; c < nchunk; ++c)
-        s += partial[((long long)c * nd + d) * n + i];
-    out[(long long)i * ld + off + (d - d0)] = scale * s;
+    for (int k = 0; k < m; ++k)
+        s += partial[(long long)k * nd * n];
+    out[(long long)i * (pos ? 3 : a.ks) + (pos ? d : d - 3)] = a.scale * s;
 }
 
 } // namespace stkp2p
