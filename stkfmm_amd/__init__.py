@@ -144,11 +144,20 @@ def get_kernel_name(kernel):
     return buf.value.decode()
 
 
+# answers of the library's fixed kernel table, kept because a small sum would spend a quarter of its time
+# asking for them
+_UKERS, _DIMS = {}, {}
+
+
 def get_uker(kernel, p2p):
     """Micro-kernel evaluated for (KERNEL, PPKERNEL) (Lib/src/FMMData.cpp:261-268)."""
-    uk = ctypes.c_int(-1)
-    _check(lib().stkfmm_get_uker(int(kernel), int(p2p), ctypes.byref(uk)))
-    return UKER(uk.value)
+    key = (int(kernel), int(p2p))
+    found = _UKERS.get(key)
+    if found is None:
+        uk = ctypes.c_int(-1)
+        _check(lib().stkfmm_get_uker(key[0], key[1], ctypes.byref(uk)))
+        found = _UKERS[key] = UKER(uk.value)
+    return found
 
 
 def get_s2m_uker(kernel, double_layer=False):
@@ -176,9 +185,13 @@ def get_m2t_uker(kernel):
 
 def uker_dims(uker):
     """(source dim, target dim) of a micro-kernel."""
-    ks, kt = ctypes.c_int(), ctypes.c_int()
-    _check(lib().stkfmm_uker_dims(int(uker), ctypes.byref(ks), ctypes.byref(kt)))
-    return ks.value, kt.value
+    uk = int(uker)
+    found = _DIMS.get(uk)
+    if found is None:
+        ks, kt = ctypes.c_int(), ctypes.c_int()
+        _check(lib().stkfmm_uker_dims(uk, ctypes.byref(ks), ctypes.byref(kt)))
+        found = _DIMS[uk] = (ks.value, kt.value)
+    return found
 
 
 def device_info():
@@ -190,14 +203,19 @@ def device_info():
 
 # ---- host (numpy) entry: STKFMM::evaluateKernel ------------------------------------------------------
 
-def _host_arr(a, n, k, name, writable=False):
+def _host_addr(a, n, k, name, writable=False):
+    """The address of a checked host array."""
     if not isinstance(a, np.ndarray) or a.dtype != np.float64 or not a.flags.c_contiguous:
         raise ArgumentError(f"{name}: expected a C-contiguous float64 numpy array")
     if writable and not a.flags.writeable:
         raise ArgumentError(f"{name}: array is read-only")
     if a.size != n * k:
         raise ArgumentError(f"{name}: expected {n}x{k} values, got {a.size}")
-    return a.ctypes.data_as(_capi.dptr)
+    return a.ctypes.data
+
+
+def _host_arr(a, n, k, name, writable=False):
+    return ctypes.cast(_host_addr(a, n, k, name, writable), _capi.dptr)
 
 
 def evaluate_kernel(kernel, n_threads, p2p, src_coord, src_value, trg_coord, trg_value, precision=PREC.FP64):
@@ -210,11 +228,11 @@ def evaluate_kernel(kernel, n_threads, p2p, src_coord, src_value, trg_coord, trg
     ks, kt = uker_dims(uk)
     ns = src_coord.size // 3
     nt = trg_coord.size // 3
-    a = _host_arr(src_coord, ns, 3, "src_coord")
-    b = _host_arr(src_value, ns, ks, "src_value")
-    c = _host_arr(trg_coord, nt, 3, "trg_coord")
-    d = _host_arr(trg_value, nt, kt, "trg_value", writable=True)
-    _check(lib().stkfmm_p2p_eval(int(kernel), int(p2p), int(precision), ns, a, b, nt, c, d))
+    a = _host_addr(src_coord, ns, 3, "src_coord")
+    b = _host_addr(src_value, ns, ks, "src_value")
+    c = _host_addr(trg_coord, nt, 3, "trg_coord")
+    d = _host_addr(trg_value, nt, kt, "trg_value", writable=True)
+    _check(_capi.by_address("stkfmm_p2p_eval")(int(kernel), int(p2p), int(precision), ns, a, b, nt, c, d))
     return trg_value
 
 
@@ -252,11 +270,11 @@ def ker_eval(uker, r_src, v_src, r_trg, v_trg, dof=1):
     """Ker_t-shaped micro-kernel entry on host arrays: v_trg += ScaleFactor * sum (FP64)."""
     ks, kt = uker_dims(uker)
     ns, nt = r_src.size // 3, r_trg.size // 3
-    a = _host_arr(r_src, ns, 3, "r_src")
-    b = _host_arr(v_src, ns, ks, "v_src")
-    c = _host_arr(r_trg, nt, 3, "r_trg")
-    d = _host_arr(v_trg, nt, kt, "v_trg", writable=True)
-    _check(lib().stkfmm_ker_eval(int(uker), a, ns, b, int(dof), c, nt, d))
+    a = _host_addr(r_src, ns, 3, "r_src")
+    b = _host_addr(v_src, ns, ks, "v_src")
+    c = _host_addr(r_trg, nt, 3, "r_trg")
+    d = _host_addr(v_trg, nt, kt, "v_trg", writable=True)
+    _check(_capi.by_address("stkfmm_ker_eval")(int(uker), a, ns, b, int(dof), c, nt, d))
     return v_trg
 
 
@@ -357,16 +375,36 @@ def wall_evaluate(kernel, src_coord, src_value, trg_coord, trg_value, precision=
 
 # ---- device (torch) entries ----------------------------------------------------------------------
 
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
 def _stream_handle(stream):
+    """Handle of a torch stream, or of the current one."""
+    if stream is not None:
+        return stream.cuda_stream
     torch = _torch()
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    try:  # the current stream without a stream object around it (8 us)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:  # another torch
+        return torch.cuda.current_stream().cuda_stream
+
+
+def _dev_rows(t, n, k, name):
+    """Validate a contiguous float64 CUDA tensor of n rows and k columns."""
+    torch = _torch()
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float64 and t.dim() == 2
+            and t.shape[0] == n and t.shape[1] == k and t.is_contiguous()):
+        return
+    _dev2d(t, n, k, name)
+    raise ArgumentError(f"{name}: expected a contiguous ({n}, {k}) tensor")
 
 
 def _dev2d(t, n, k, name, writable=False):
@@ -376,17 +414,17 @@ def _dev2d(t, n, k, name, writable=False):
         raise ArgumentError(f"{name}: expected a float64 CUDA tensor")
     if t.dim() != 2 or t.shape[0] < n or t.shape[1] < k:
         raise ArgumentError(f"{name}: expected shape >= ({n}, {k}), got {tuple(t.shape)}")
-    if n > 0 and (t.stride(0) < 0 or t.stride(1) < 0):
+    if n > 0 and min(t.stride()) < 0:
         raise ArgumentError(f"{name}: negative strides")
     return t
 
 
 def _sarr(t):
-    return StkArray(t.data_ptr(), t.stride(0), t.stride(1))
+    return StkArray(t.data_ptr(), *t.stride())
 
 
 def _oarr(t):
-    return StkOutArray(t.data_ptr(), t.stride(0), t.stride(1))
+    return StkOutArray(t.data_ptr(), *t.stride())
 
 
 def p2p_device(kernel, p2p, src_coord, src_value, trg_coord, trg_value, precision=PREC.FP64, stream=None,
@@ -400,9 +438,7 @@ def p2p_device(kernel, p2p, src_coord, src_value, trg_coord, trg_value, precisio
     ns, nt = src_coord.shape[0], trg_coord.shape[0]
     for t, n, k, nm in ((src_coord, ns, 3, "src_coord"), (src_value, ns, ks, "src_value"),
                         (trg_coord, nt, 3, "trg_coord"), (trg_value, nt, kt, "trg_value")):
-        _dev2d(t, n, k, nm)
-        if not t.is_contiguous() or t.shape[1] != k or t.shape[0] != n:
-            raise ArgumentError(f"{nm}: expected a contiguous ({n}, {k}) tensor")
+        _dev_rows(t, n, k, nm)
     entry = lib().stkfmm_p2p_eval_device_noalloc if no_alloc else lib().stkfmm_p2p_eval_device
     _check(entry(int(kernel), int(p2p), int(precision), ns, src_coord.data_ptr(), src_value.data_ptr(), nt,
                  trg_coord.data_ptr(), trg_value.data_ptr(), _stream_handle(stream)))
@@ -445,9 +481,7 @@ def vjp_device(uker, src_coord, src_value, trg_coord, w, precision=PREC.FP64, ne
     ns, nt = src_coord.shape[0], trg_coord.shape[0]
     for t, n, k, nm in ((src_coord, ns, 3, "src_coord"), (src_value, ns, ks, "src_value"),
                         (trg_coord, nt, 3, "trg_coord"), (w, nt, kt, "w")):
-        _dev2d(t, n, k, nm)
-        if not t.is_contiguous() or t.shape[1] != k or t.shape[0] != n:
-            raise ArgumentError(f"{nm}: expected a contiguous ({n}, {k}) tensor")
+        _dev_rows(t, n, k, nm)
     dev = src_coord.device
     gsv = torch.empty((ns, ks), dtype=torch.float64, device=dev) if need[0] else None
     gsc = torch.empty((ns, 3), dtype=torch.float64, device=dev) if need[1] else None
@@ -699,6 +733,7 @@ class Plan:
         self.precision = PREC(int(precision))
         self.n_src, self.n_trg = int(n_src), int(n_trg)
         self.ks, self.kt = uker_dims(uker)
+        self._fused = self.uker == UKER.STOKES_PVEL_FUSED
         self._keep = None
 
     @classmethod
@@ -733,11 +768,11 @@ class Plan:
         return a.value, b.value, n.value
 
     def _args(self, src_coord, src_value, trg_coord, trg_value, src_value2, perm):
-        ks1 = 4 if self.uker == UKER.STOKES_PVEL_FUSED else self.ks
+        ks1 = 4 if self._fused else self.ks
         _dev2d(src_coord, self.n_src, 3, "src_coord")
         _dev2d(src_value, self.n_src, ks1, "src_value")
         _dev2d(trg_coord, self.n_trg, 3, "trg_coord")
-        if self.uker == UKER.STOKES_PVEL_FUSED:
+        if self._fused:
             if src_value2 is None:
                 raise ArgumentError("STOKES_PVEL_FUSED needs src_value2 (double-layer values)")
             _dev2d(src_value2, self.n_src, 9, "src_value2")
@@ -751,8 +786,9 @@ class Plan:
                 raise ArgumentError("perm: values outside the output rows")
         else:
             _dev2d(trg_value, self.n_trg, self.kt, "trg_value")
-        sv2 = _sarr(src_value2) if src_value2 is not None else _sarr(src_value)
-        args = (_sarr(src_coord), _sarr(src_value), sv2, _sarr(trg_coord), _oarr(trg_value))
+        sv = _sarr(src_value)
+        sv2 = _sarr(src_value2) if src_value2 is not None else sv
+        args = (_sarr(src_coord), sv, sv2, _sarr(trg_coord), _oarr(trg_value))
         return args, (None if perm is None else perm.data_ptr())
 
     def execute(self, src_coord, src_value, trg_coord, trg_value, src_value2=None, perm=None, stream=None):

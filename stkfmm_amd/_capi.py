@@ -136,5 +136,21 @@ def lib():
     return _lib
 
 
+_BY_ADDRESS = {}
+
+
+def by_address(name):
+    """An entry of the library that takes its arrays as plain addresses (a typed pointer costs more than 1 us
+    to make)."""
+    f = _BY_ADDRESS.get(name)
+    if f is None:
+        declared = getattr(lib(), name)
+        f = lib()[name]  # a function object of its own
+        f.restype = declared.restype
+        f.argtypes = [c_void_p if t is dptr else t for t in declared.argtypes]
+        _BY_ADDRESS[name] = f
+    return f
+
+
 def last_error():
     return lib().stkfmm_last_error().decode()

@@ -11,16 +11,16 @@ import torch
 
 from . import PREC, UKER, uker_device, uker_dims, vjp_device
 
-_ADJOINT_UKERS = (UKER.LAPLACE_P, UKER.LAPLACE_PGRAD, UKER.STOKES_VEL, UKER.STOKES_REGVEL, UKER.RPY_U,
-                  UKER.RPY_ULAPU, UKER.STK_ULAPU, UKER.STOKES_PVEL, UKER.STOKES_DOUBLEPVEL, UKER.STOKES_PVEL_FUSED)
+_ADJOINT_UKERS = frozenset(int(u) for u in (
+    UKER.LAPLACE_P, UKER.LAPLACE_PGRAD, UKER.STOKES_VEL, UKER.STOKES_REGVEL, UKER.RPY_U, UKER.RPY_ULAPU,
+    UKER.STK_ULAPU, UKER.STOKES_PVEL, UKER.STOKES_DOUBLEPVEL, UKER.STOKES_PVEL_FUSED))
 
 
 class P2PFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, uker, precision, src_coord, src_value, trg_coord):
-        uker = UKER(int(uker))
         if uker not in _ADJOINT_UKERS:
-            raise ValueError(f"no adjoint kernel for {uker.name}")
+            raise ValueError(f"no adjoint kernel for {UKER(int(uker)).name}")
         _, kt = uker_dims(uker)
         sc, sv, tc = src_coord.contiguous(), src_value.contiguous(), trg_coord.contiguous()
         out = torch.zeros((tc.shape[0], kt), dtype=torch.float64, device=tc.device)
