@@ -47,6 +47,15 @@ namespace stkp2p {
 // MASK: 0 unless r2 > 0 -- a select after the refinement (a NaN r2 must give 0 like the reference's
 // mask, and a Newton step turns any seed into NaN when r2 is NaN).  MASK = false drops the select,
 // for pairs known to have r2 > 0 (the result is then the same).
+// The mask zeroes the high word only, one select for two (about 2.5 of LapPGrad's 100 cycles a pair): at r2 = 0
+// the seed is infinite and the Newton step 0 * inf, whose NaN has a zero low word, and so has the NaN of a
+// NaN coordinate; only a NaN with payload bits there leaves a denormal (below 1e-308) instead of 0.
+__device__ __forceinline__ double masked_f64(double y, double r2) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, y);
+    const unsigned hi = (r2 > 0.0) ? (unsigned)(b >> 32) : 0u;
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | (unsigned)b);
+}
+
 template <bool MASK = true>
 __device__ __forceinline__ double rsqrt_f64(double r2) {
     double y = __builtin_amdgcn_rsq(r2);
@@ -57,7 +66,7 @@ __device__ __forceinline__ double rsqrt_f64(double r2) {
         y = __builtin_fma(y, e, y);
     }
     if constexpr (MASK)
-        return (r2 > 0.0) ? y : 0.0;
+        return masked_f64(y, r2);
     else
         return y;
 }
@@ -77,7 +86,7 @@ __device__ __forceinline__ double twice_rsqrt_f64(double r2) {
     }
     const double w = y * __builtin_fma(-r2, y * y, 3.0);
     if constexpr (MASK)
-        return (r2 > 0.0) ? w : 0.0;
+        return masked_f64(w, r2);
     else
         return w;
 }
@@ -268,14 +277,29 @@ struct UkLaplacePGrad {
 // FP32 form stays finite down to r ~ 1e-12 (1/r^5 overflows FP32 below r ~ 2e-8).
 struct UkLaplaceDipolePGrad {
     static constexpr int KS = 3, KS1 = 3, KL = 3, KT = 4;
-    static constexpr bool UNMASKED_EVAL = true;
+    static constexpr bool UNMASKED_EVAL = true, POST_BY_PRECISION = true;
     static constexpr unsigned SRC_SCALE_MASK = 0x7u;
     __host__ __device__ static constexpr int deg(int k) { return k == 0 ? 1 : 2; }
     __host__ __device__ static constexpr double post(int k) { return ((void)k, 1.0); }
+    // FP64 takes w = 2/r: 8 times its value
+    template <int PREC>
+    __host__ __device__ static constexpr double post_p(int) { return PREC == 0 ? 0.125 : 1.0; }
     __device__ static void stage(const double *in, double *o) { o[0] = in[0]; o[1] = in[1]; o[2] = in[2]; }
     template <class R, bool M = true>
     __device__ static void eval(R *u, R dx, R dy, R dz, const R *f) {
         R r2 = dx * dx + dy * dy + dz * dz;
+        if constexpr (sizeof(R) == 8) {
+            const R w = twice_rsqrt_f64<M>(r2);
+            const R w2 = w * w;
+            const R w3 = w2 * w;
+            const R c = f[0] * dx + f[1] * dy + f[2] * dz;
+            const R k = R(-0.75) * (c * w2);
+            u[0] += c * w3;
+            u[1] += (k * dx + f[0]) * w3;
+            u[2] += (k * dy + f[1]) * w3;
+            u[3] += (k * dz + f[2]) * w3;
+            return;
+        }
         const auto rs = pair_rsqrt<M>(r2);
         R rinv = rs.s, rinv2 = rs.s2;
         R rinv3 = rinv2 * rinv;
@@ -534,16 +558,22 @@ struct UkStokesPVel {
 //   FP32: Horner in dx, dy, dz reusing dz^2 of r^2; staged g0..g5, tr D.
 //   FP64: with z^2 = r^2 - x^2 - y^2, -3 Q = g2 r^2 + rest, rest = x ((g0 - g2) x + g3 y + g4 z) +
 //         y ((g1 - g2) y + g5 z), so t = g2 + rest/r^2 -- one operation fewer; staged g0 - g2,
-//         g1 - g2, g2, g3, g4, g5, tr D.  (In FP32 the split adds rounding of size |g2| to t, measured
+//         g1 - g2, g2, g3, g4, g5, tr D (sym_p); and w = 2/r with the quadratic form's coefficients / 4, so that
+//         t = g2 + rest w^2, and w^3 = 8/r^3 (post() / 8).  (In FP32 the split adds rounding of size |g2| to t, measured
 //         up to 3x the Horner form's error on clustered U-lists, so FP32 keeps the Horner form.)
 struct UkStokesDoublePVel {
     static constexpr int KS = 9, KS1 = 9, KL = 7, KT = 4;
-    static constexpr bool UNMASKED_EVAL = true, STAGE_BY_PRECISION = true;
+    static constexpr bool UNMASKED_EVAL = true, STAGE_BY_PRECISION = true, POST_BY_PRECISION = true;
     static constexpr unsigned SRC_SCALE_MASK = 0x1FFu;
     __host__ __device__ static constexpr int deg(int k) { return k == 0 ? 2 : 1; }
     __host__ __device__ static constexpr double post(int k) { return k == 0 ? 2.0 : 1.0; }
     template <int PREC>
-    __host__ __device__ static void stage_p(const double *in, double *o) {
+    __host__ __device__ static constexpr double post_p(int k) {
+        return PREC == 0 ? 0.125 * post(k) : post(k);
+    }
+    // the quadratic form and tr D
+    template <int PREC>
+    __host__ __device__ static void sym_p(const double *in, double *o) {
         const double g0 = -3.0 * in[0], g1 = -3.0 * in[4], g2 = -3.0 * in[8];
         o[0] = (PREC == 0) ? g0 - g2 : g0;
         o[1] = (PREC == 0) ? g1 - g2 : g1;
@@ -553,27 +583,35 @@ struct UkStokesDoublePVel {
         o[5] = -3.0 * (in[5] + in[7]);
         o[6] = in[0] + in[4] + in[8];
     }
-    // -3 r.D.r / r^2 from the first six staged values (the layout of stage_p for R's precision), z2 = dz^2
-    template <class R>
-    __device__ static R t_of(R dx, R dy, R dz, R z2, R rinv2, const R *g) {
-        if constexpr (sizeof(R) == 8) {
-            const R a1 = g[0] * dx + g[3] * dy + g[4] * dz;
-            const R a2 = g[1] * dy + g[5] * dz;
-            return (dx * a1 + dy * a2) * rinv2 + g[2];
-        } else {
-            const R a1 = g[0] * dx + g[3] * dy + g[4] * dz;
-            const R a2 = g[1] * dy + g[5] * dz;
-            return (dx * a1 + (dy * a2 + g[2] * z2)) * rinv2;
-        }
+    template <int PREC>
+    __host__ __device__ static void stage_p(const double *in, double *o) {
+        sym_p<PREC>(in, o);
+        if constexpr (PREC == 0)
+            for (int k = 0; k < 6; ++k)
+                if (k != 2) o[k] *= 0.25;
     }
     template <class R, bool M = true>
     __device__ static void eval(R *u, R dx, R dy, R dz, const R *g) {
         const R z2 = dz * dz;
         R r2 = dx * dx + (dy * dy + z2);
+        const R a1 = g[0] * dx + g[3] * dy + g[4] * dz;
+        const R a2 = g[1] * dy + g[5] * dz;
+        if constexpr (sizeof(R) == 8) {
+            const R w = twice_rsqrt_f64<M>(r2);
+            const R w2 = w * w;
+            const R w3 = w2 * w;
+            const R t = (dx * a1 + dy * a2) * w2 + g[2];
+            const R q = t * w3;
+            u[0] += (t + g[6]) * w3;
+            u[1] += dx * q;
+            u[2] += dy * q;
+            u[3] += dz * q;
+            return;
+        }
         const auto rs = pair_rsqrt<M>(r2);
         R rinv = rs.s, rinv2 = rs.s2;
         R rinv3 = rinv2 * rinv;
-        R t = t_of(dx, dy, dz, z2, rinv2, g);
+        R t = (dx * a1 + (dy * a2 + g[2] * z2)) * rinv2;
         R q = t * rinv3;
         u[0] += (t + g[6]) * rinv3;
         u[1] += dx * q;
@@ -610,7 +648,7 @@ struct UkStokesPVelFused {
     template <int PREC>
     __host__ __device__ static void stage_p(const double *in, double *o) {
         double d[7];
-        UkStokesDoublePVel::stage_p<PREC>(in + 4, d);
+        UkStokesDoublePVel::sym_p<PREC>(in + 4, d);
         o[0] = in[0]; o[1] = in[1]; o[2] = in[2];
         if constexpr (PREC == 0) {
             o[0] = 0.125 * in[0]; o[1] = 0.125 * in[1]; o[2] = 0.125 * in[2];
@@ -684,6 +722,20 @@ struct UkStokesRegVel {
     template <class R, bool M = true>
     __device__ static void eval(R *u, R dx, R dy, R dz, const R *f) {
         const R reg2 = f[3];
+        if constexpr (sizeof(R) == 8) {
+            // (rho2 + eps^2)/rho^3 = 1/rho + eps^2/rho^3
+            const R s = rsqrt_f64<M>(dx * dx + (dy * dy + (dz * dz + reg2)));
+            const R s3 = (s * s) * s;
+            const R a = reg2 * s3 + s;
+            const R b = (f[0] * dx + f[1] * dy + f[2] * dz) * s3;
+            u[0] += f[0] * a;
+            u[0] += dx * b;
+            u[1] += f[1] * a;
+            u[1] += dy * b;
+            u[2] += f[2] * a;
+            u[2] += dz * b;
+            return;
+        }
         R r2 = dx * dx + dy * dy + dz * dz + reg2;
         const auto rs = pair_rsqrt<M>(r2);
         R rinv3 = rs.s2 * rs.s;
