@@ -22,66 +22,65 @@
 namespace stkp2p {
 
 
-// out(perm[i], k) += scale * sum over the tile's slots of partial[slot][k][i]; one workgroup per
-// (tile, group of KG output components k = KG*blockIdx.y + c), blockDim = 64*T.  Each (target, k) sums
-// its slots in slot order, so the result does not depend on the grid shape.  KG = 4 for kernels with
-// more than 4 outputs over at least 2048 tiles: the components of a group are summed side by side, so
-// that their loads are in flight together (one workgroup per component left the 16-output kernels
-// with ~10^5 one-wave workgroups, latency-bound: reduce 0.178 -> 0.141 ms on a 262,144-point
-// U-list); KG = 1 otherwise, where grouping left too few workgroups (the 4-output PVel U-list reduce
-// 0.106 -> 0.119 ms; 65,536-target direct sums of 512 tiles and ~64 slots each slower).
-template <int KG>
-__global__ void __launch_bounds__(256) p2p_reduce_kernel(ReduceArgs a) {
-    const Tile tl = a.tiles[blockIdx.x];
+// out(perm[i], k) += scale * sum over the tile's slots of partial[slot][k][i], NK components from k0 for one
+// target: each (target, k) sums its slots in slot order, so the result does not depend on the grid shape.  The
+// NK * UNROLL loads of a step and the old outputs are in flight together.
+template <int NK, int UNROLL>
+__device__ __forceinline__ void reduce_slots(const ReduceArgs &a, const Tile &tl, int k0) {
     const int i = threadIdx.x;
     if (i >= tl.trg_count)
         return;
-    const int k0 = blockIdx.y * KG;
-    const int nk = min(KG, a.kt - k0);
+    const int nk = min(NK, a.kt - k0);
     const long long row = tl.trg_begin + i;
     const long long o = a.perm ? (long long)a.perm[row] : row;
+    double *const out = a.out.p + o * a.out.s + k0 * a.out.fs;
     const long long step = (long long)a.kt * a.tt;
     const double *__restrict__ part = a.partial + (long long)k0 * a.tt + i;
-    double sum[KG];
+    double sum[NK], old[NK];
 #pragma unroll
-    for (int c = 0; c < KG; ++c)
+    for (int c = 0; c < NK; ++c) {
         sum[c] = 0.0;
-    // unrolled so that the loads of several slots are in flight together (the adds keep slot order)
-    constexpr int kSlotUnroll = KG == 1 ? 4 : 2;
-#pragma unroll kSlotUnroll
+        old[c] = (c < nk) ? out[c * a.out.fs] : 0.0;
+    }
+#pragma unroll UNROLL
     for (int slot = tl.slot_begin; slot < tl.slot_end; ++slot) {
         const double *__restrict__ q = part + slot * step;
 #pragma unroll
-        for (int c = 0; c < KG; ++c)
+        for (int c = 0; c < NK; ++c)
             if (c < nk)
                 sum[c] += q[(long long)c * a.tt];
     }
 #pragma unroll
-    for (int c = 0; c < KG; ++c)
+    for (int c = 0; c < NK; ++c)
         if (c < nk)
-            a.out.p[o * a.out.s + (k0 + c) * a.out.fs] += a.scale * sum[c];
+            out[c * a.out.fs] = old[c] + a.scale * sum[c];
 }
 
-// out(perm[i], k) += scale * (slot sums) for every k of target i in one thread: the same sums in the
-// same order as p2p_reduce_kernel (bitwise the same result), one workgroup per tile, tiles dealt to
+// one workgroup per (tile, group of KG components), the groups of a tile one after another on one XCD, so that
+// the lines of its output rows are read and written once (16 outputs of 262,144 targets 140 -> 122 us, 4 of 10^5
+// expansion targets 36.5 -> 25.7).  KG = 4 for kernels with
+// more than 4 outputs over at least 2048 tiles: the components of a group are summed side by side, so
+// that their loads are in flight together (one workgroup per component left the 16-output kernels
+// with ~10^5 one-wave workgroups, latency-bound); KG = 1 otherwise, where grouping left too few workgroups (the
+// 4-output PVel U-list reduce 0.106 -> 0.119 ms; 65,536-target direct sums of 512 tiles and ~64 slots each slower).
+template <int KG>
+__global__ void __launch_bounds__(256) p2p_reduce_kernel(ReduceArgs a) {
+    const int groups = (a.kt + KG - 1) / KG;
+    const int u = xcd_unit(blockIdx.x, a.n_tiles * groups);
+    if (u < 0)
+        return;
+    reduce_slots<KG, KG == 1 ? 16 : 4>(a, a.tiles[u / groups], u % groups * KG);
+}
+
+// every component of a target in one thread: one workgroup per tile, tiles dealt to
 // the XCDs in contiguous runs (the scattered rows of neighbouring tiles then share one L2)
 __global__ void __launch_bounds__(256) p2p_reduce_rows_kernel(ReduceArgs a) {
     const int ti = xcd_unit(blockIdx.x, a.n_tiles);
     if (ti < 0)
         return;
     const Tile tl = a.tiles[ti];
-    const int i = threadIdx.x;
-    if (i >= tl.trg_count)
-        return;
-    const long long row = tl.trg_begin + i;
-    const long long o = a.perm ? (long long)a.perm[row] : row;
-    for (int k = 0; k < a.kt; ++k) {
-        double s = 0.0;
-#pragma unroll 4
-        for (int slot = tl.slot_begin; slot < tl.slot_end; ++slot)
-            s += a.partial[((long long)slot * a.kt + k) * a.tt + i];
-        a.out.p[o * a.out.s + k * a.out.fs] += a.scale * s;
-    }
+    for (int k0 = 0; k0 < a.kt; k0 += 4)
+        reduce_slots<4, 4>(a, tl, k0);
 }
 
 __global__ void fill_int_kernel(int *p, int n, int value) {
@@ -243,13 +242,19 @@ int record_words(int uk, int prec) {
     return (o && (prec == 0 || prec == 1)) ? o->words[prec] : -1;
 }
 
-hipError_t launch_reduce(const ReduceArgs &a, hipStream_t s) {
-    if (a.n_tiles <= 0)
-        return hipSuccess;
-    if (a.kt > 4 && a.n_tiles >= 2048)
-        hipLaunchKernelGGL(p2p_reduce_kernel<4>, dim3(a.n_tiles, (a.kt + 3) / 4), dim3(a.tt), 0, s, a);
-    else
-        hipLaunchKernelGGL(p2p_reduce_kernel<1>, dim3(a.n_tiles, a.kt), dim3(a.tt), 0, s, a);
+hipError_t launch_reduce(const ReduceArgs &all, hipStream_t s) {
+    constexpr int kMaxTiles = 1 << 20; // a launch: keeps its thread count within 32 bits
+    const bool wide = all.kt > 4 && all.n_tiles >= 2048;
+    for (int t0 = 0; t0 < all.n_tiles; t0 += kMaxTiles) {
+        ReduceArgs a = all;
+        a.tiles += t0;
+        a.n_tiles = std::min(kMaxTiles, all.n_tiles - t0);
+        const dim3 grid((unsigned)xcd_grid(a.n_tiles * (wide ? (a.kt + 3) / 4 : a.kt)));
+        if (wide)
+            hipLaunchKernelGGL(p2p_reduce_kernel<4>, grid, dim3(a.tt), 0, s, a);
+        else
+            hipLaunchKernelGGL(p2p_reduce_kernel<1>, grid, dim3(a.tt), 0, s, a);
+    }
     return hipGetLastError();
 }
 
