@@ -362,13 +362,13 @@ static void group_tiles(int n, int TT, bool pieces, std::vector<int> &counts) {
 // sizes a direct sum's 32-bit indices cover
 static bool direct_sizes(int n_src, int n_trg) { return n_src <= (1 << 30) && n_trg <= (1 << 30); }
 // direct sums whose entry orders the points (or whose sizes one launch does not cover)
-static bool direct_sorts_points(int n_src, int n_trg) {
-    return (n_src >= kDirectSortMin && n_trg >= kDirectSortMin) || !direct_sizes(n_src, n_trg);
+static bool direct_sorts_points(int prec, int n_src, int n_trg) {
+    return direct_ordered_pays(prec, n_src, n_trg) || !direct_sizes(n_src, n_trg);
 }
 
 // direct sums that are one launch
 static bool direct_in_one_call(int uk, int prec, int n_src, int n_trg) {
-    return !direct_sorts_points(n_src, n_trg) && direct_in_one_launch(prec, uk);
+    return !direct_sorts_points(prec, n_src, n_trg) && direct_in_one_launch(prec, uk);
 }
 
 extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision, int n_src, int n_trg,
@@ -390,6 +390,22 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     stkfmm_tune tn{};
     if (tune)
         tn = *tune;
+    const stkfmm_tune no_tune{};
+    const bool untuned = std::memcmp(&tn, &no_tune, sizeof(tn)) == 0;
+    // one direct sum over a plain list
+    const bool single = n_groups == 1 && !grp_level && grp_rng_ptr[0] >= 0 &&
+                        (long long)grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && rng_src_begin && rng_src_end;
+    // A large untuned FP64 one orders its points: PVel 65,536^2 3.90 -> 3.65 ms, PVelGrad 8.06 -> 7.82, Laplace
+    // potential 1.97 -> 1.82.  Staged in LDS: the scalar-broadcast records of the device entries (direct_plan) take
+    // 3.58 ms, but draw more power, and the adjoint pass that follows in a training step then runs at a lower
+    // clock (forward and adjoint in turn 12.17 ms as given, 12.04 ordered in LDS, 12.39 with the records).
+    // (Mixed mode keeps the order it is given: its FP32 sums depend on it.)
+    if (untuned && single && precision == STKFMM_PREC_FP64 &&
+        direct_ordered_pays(precision, (long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]],
+                            (long long)grp_trg_end[0] - grp_trg_begin[0])) {
+        tn.sort_points = 1;
+        tn.targets_per_lane = 2;
+    }
     // default targets per lane: 2, and 1 in mixed mode for the family members with many outputs or
     // much per-pair state, whose two-target loops run at lower occupancy: 262,144-point U-list, item
     // kernel + reduce (ms), T = 2 -> 1: PVelGrad 2.25 -> 2.03, LapQPGradGrad 2.34 -> 2.13,
@@ -673,11 +689,8 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     (void)hipGetDevice(&p->device);
 
     // A single untuned direct sum below the sizes that pay for ordered points: one launch instead of queue
-    // reset, item kernel and reduce (above, the item kernel is the faster one: 65,536^2 PVel FP64 as given
-    // 4.0 against 4.3 ms).  The item list above stays for stkfmm_plan_stats.
-    const stkfmm_tune no_tune{};
-    if (n_groups == 1 && !grp_level && std::memcmp(&tn, &no_tune, sizeof(tn)) == 0 && p->n_items > 0 &&
-        grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && direct_in_one_call(uk, precision, n_src, n_trg)) {
+    // reset, item kernel and reduce.  The item list above stays for stkfmm_plan_stats.
+    if (untuned && single && p->n_items > 0 && direct_in_one_call(uk, precision, n_src, n_trg)) {
         const int r0 = grp_rng_ptr[0];
         p->direct = true;
         p->dt_begin = grp_trg_begin[0];
@@ -1127,7 +1140,7 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
     if (direct_in_one_call(uk, prec, n_src, n_trg)) {
         int n_cu = 0;
         double *partial = nullptr;
-        if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
+        if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial, store)))
             return rc;
         const DirectLayout l = direct_layout_uk(uk, prec, direct_targets_per_lane(prec, kt, n_trg), n_src, n_trg, n_cu);
         DirectArgs a = direct_args(uk, n_src, n_trg, DArr{sc, 3, 1}, DArr{sv, ks, 1}, DArr{sv + ks1, ks, 1},
@@ -1271,7 +1284,7 @@ int wall_device(unsigned kernel, const double *sc, const double *sv, int n, cons
                 hipStream_t s, bool store = false) {
     int n_cu = 0, rc;
     double *partial = nullptr;
-    if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial)))
+    if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial, store)))
         return rc;
     const int ks = kernel == STKFMM_KERNEL_Stokes ? 3 : 4, kt = kernel == STKFMM_KERNEL_Stokes ? 3 : 6;
     DirectArgs a{};

@@ -229,8 +229,14 @@ inline int direct_targets_per_lane(int prec, int kt, int n_trg) {
 // the result apart, and keep the item kernels.  tests/test_gpu_direct_launch.py holds all others to it.
 inline bool direct_in_one_launch(int prec, int uk) { return prec == 0 || (uk != 15 && uk != 17 && uk != 22); }
 // Direct sums with at least this many sources and targets order their points (sort_points) in the
-// plan-based entries.
+// plan-based entries: in mixed mode, whose far form they then reach, from there on; in FP64, which gains the
+// unmasked form only, from 2^29 pairs (one launch against ordered points, us: 16,384^2 PVel 245 and 335,
+// PVelGrad 574 and 559; 24,001^2 522 and 588, 1,115 and 1,118; 32,768^2 969 and 983, 1,994 and 1,970;
+// 40,009 x 30,011 1,126 and 1,068, 2,406 and 2,187).
 constexpr int kDirectSortMin = 16384;
+inline bool direct_ordered_pays(int prec, long long n_src, long long n_trg) {
+    return n_src >= kDirectSortMin && n_trg >= kDirectSortMin && (prec != 0 || n_src * n_trg >= 1LL << 29);
+}
 
 // lanes per target of a tile of n targets (log2): the largest power of two, at most 16, that still
 // fits the tile's 64*T lanes
@@ -280,7 +286,7 @@ hipError_t items_sgpr_occupancy(int uk, int prec, int T, int *blocks_per_cu);
 int uker_run(int uk);
 // device memory for the chunks' partial sums of the direct-sum entries on the current device
 // (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
-int direct_partial_ptr(double **out);
+int direct_partial_ptr(double **out, bool host);
 // out shares memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
 // the item and reduce kernels do
 bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt);

@@ -57,8 +57,8 @@ __device__ __forceinline__ void reduce_slots(const ReduceArgs &a, const Tile &tl
 }
 
 // one workgroup per (tile, group of KG components), the groups of a tile one after another on one XCD, so that
-// the lines of its output rows are read and written once (16 outputs of 262,144 targets 140 -> 122 us, 4 of 10^5
-// expansion targets 36.5 -> 25.7).  KG = 4 for kernels with
+// the lines of its output rows are read and written once (16 outputs of 262,144 targets 140 -> 122 us, 4 of the
+// expansion surfaces of 262,144 clustered points 36.5 -> 25.7).  KG = 4 for kernels with
 // more than 4 outputs over at least 2048 tiles: the components of a group are summed side by side, so
 // that their loads are in flight together (one workgroup per component left the 16-output kernels
 // with ~10^5 one-wave workgroups, latency-bound); KG = 1 otherwise, where grouping left too few workgroups (the

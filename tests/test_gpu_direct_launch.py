@@ -131,3 +131,35 @@ def test_output_over_an_input():
     S.wall_device(S.KERNEL.Stokes, d_z, d_f, d_z, d_f)
     l2, mx = O.max_error(host(d_f), f + O.wall(int(S.KERNEL.Stokes), z, f, z))
     assert l2 < FP64_TOL and mx < FP64_TOL, ("wall", l2, mx)
+
+
+@pytest.mark.parametrize("ns,nt,same", [(16384, 16384, False), (16384, 32767, False), (16384, 32768, False),
+                                        (23170, 23170, True), (23171, 23171, True)])
+@pytest.mark.parametrize("uk", [0, 8, 13, 15])
+def test_fp64_sums_where_ordered_points_begin(uk, ns, nt, same):
+    """One launch below 2^29 pairs, ordered points from there: the untuned plan and the device entry against the
+    item kernels on the points as given."""
+    uk = S.UKER(uk)
+    say(f"direct or ordered uk={uk.name} ns={ns} nt={nt}")
+    ks, kt = S.uker_dims(uk)
+    rng = np.random.default_rng(ns + nt)
+    src = rng.random((ns, 3))
+    d_src = layout(src, not same)
+    d_trg = d_src if same else layout(rng.random((nt, 3)) ** 2, False)
+    d_val = layout(source_values(int(uk), ns, rng), True)
+    v1, v2 = (d_val[:, :4], d_val[:, 4:]) if uk == S.UKER.STOKES_PVEL_FUSED else (d_val, None)
+    perm = rng.permutation(nt).astype(np.int32)
+    d_perm = to_dev(perm)
+    got = []
+    for tune in (dict(max_src_per_item=4096), None):
+        plan = S.Plan(uk, 0, ns, nt, [0], [nt], None, [0, 1], [0], [ns], tune)
+        out = zeros(nt, kt)
+        for _ in range(2):  # adds
+            plan.execute(d_src, v1, d_trg, out, src_value2=v2, perm=d_perm)
+        got.append(host(out)[perm] / 2)
+    out = zeros(nt, kt)
+    S.uker_device(uk, d_src.contiguous(), d_val.contiguous(), d_trg.contiguous(), out)
+    got.append(host(out))
+    for g in got[1:]:
+        l2, mx = O.max_error(g, got[0])
+        assert l2 < FP64_TOL and mx < FP64_TOL, (l2, mx)
