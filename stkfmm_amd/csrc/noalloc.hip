@@ -184,7 +184,8 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
     const int ks = uker_ks(uk), ks1 = uker_ks1(uk), kt = uker_kt(uk);
     const long long n_tiles = (nTrg + TT - 1) / TT;
     // the plan's chunking, or fewer and longer chunks when its partial sums do not fit
-    long long max_src = default_max_src((long long)nSrc * n_tiles, (long long)n_cu * bpc);
+    const int cut_blocks = precision == STKFMM_PREC_FP64 ? bpc : mixed_cut_blocks(uk, T, false, false);
+    long long max_src = default_max_src((long long)nSrc * n_tiles, (long long)n_cu * cut_blocks);
     long long nc = (nSrc + max_src - 1) / max_src;
     const bool limited = layout(n_tiles * nc, n_tiles, kt, TT).end > kScratchBytes;
     if (limited) {

@@ -515,7 +515,9 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         HIP_TRY(items_occupancy(uk, kernel_prec, T, &bpc), "occupancy query");
     if (bpc < 1)
         bpc = 1;
-    const int concurrent = n_cu * bpc;
+    const int cut_blocks =
+        precision == STKFMM_PREC_FP64 ? bpc : mixed_cut_blocks(uk, T, broadcast != 0, kernel_prec == kPrecMixedFar);
+    const int concurrent = n_cu * cut_blocks;
 
     long long max_src = tn.max_src_per_item;
     if (max_src <= 0 && persistent == 3) {

@@ -215,6 +215,23 @@ inline long long default_max_src(long long total_cost, long long concurrent) {
     return m > 512 ? m : 512;
 }
 
+// Workgroups per CU from which the default item size of a mixed-mode plan is counted.  Where a long source list
+// is cut decides which sources share an FP32 partial sum, and so the results' last FP32 bits: the cuts follow this
+// table (waves per SIMD of each micro-kernel, 0 to 24), not the register allocation of the build at hand.  In FP64
+// they follow the build's occupancy.
+inline int mixed_cut_blocks(int uk, int T, bool broadcast, bool far) {
+    static const char kWaves[7][26] = {
+        "7777647767757544666547476", // LDS, T = 1
+        "7755445455544432444444354", // LDS, T = 2
+        "4444224434443311322223234", // LDS, T = 4
+        "5544334444444432444444354", // LDS, T = 2, far form
+        "7777547777766544765547477", // scalar broadcast, T = 1
+        "7744324444444422433344354", // scalar broadcast, T = 2
+        "4433113334422311221122143", // scalar broadcast, T = 4
+    };
+    return 4 * (kWaves[broadcast ? (T >> 1) + 4 : (far ? 3 : T >> 1)][uk] - '0');
+}
+
 // Targets per lane of a direct sum in one launch.  FP64: two (half the LDS reads per pair), but one for
 // more than six outputs, whose two-target loops take 130-254 VGPRs (two or three waves per SIMD).
 // Mixed mode: one below 32,768 targets, else two (its FP32 partial sums follow the tiles of 64*T

@@ -150,14 +150,13 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
 
     const int lane = threadIdx.x;
     ItemCursor cur(a);
+    // uniform by construction; readfirstlane lets the compiler keep the item in SGPRs (and the
+    // scalar-broadcast variant's record reads as scalar loads)
+    int it = __builtin_amdgcn_readfirstlane(first_item(a, cur, lane));
+    if (it < 0)
+        return;
+    Item item = a.items[it];
     for (;;) {
-        // uniform by construction; readfirstlane lets the compiler keep the item in SGPRs (and the
-        // scalar-broadcast variant's record reads as scalar loads)
-        const int it = __builtin_amdgcn_readfirstlane(next_item(a, cur, lane));
-        if (it < 0)
-            break;
-
-        const Item item = a.items[it];
         const double lam = (PREC == 0) ? 1.0 : ldexp(1.0, item.level);
         // lanes per target (uniform): lane = target slot * split + sub
         const int ls = item.lsplit & (kItemWhole - 1);
@@ -464,8 +463,10 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
             }
         }
 
+        int le = lane; // what follows from it is computed here, not held in registers over the pair loops
+        asm volatile("" : "+v"(le));
         if constexpr (PREC != 0)
-            redo_nonfinite_fp64<K>(a, item, acc, ls ? sub : 0, split, tx, ty, tz, lam);
+            redo_nonfinite_fp64<K>(a, item, acc, le & (split - 1), split, tx, ty, tz, lam);
         // lanes that share a target add their partial sums (butterfly over the low ls lane bits)
         for (int off = 1; off < split; off <<= 1) {
 #pragma unroll
@@ -474,11 +475,20 @@ __attribute__((amdgpu_waves_per_eu(ItemMinWaves<UK, PREC>::value))) p2p_items_ke
                 for (int k = 0; k < NA; ++k)
                     acc[t][k] += __shfl_xor(acc[t][k], off);
         }
+        const int ticket = request_item(a, cur, le);
         double out[T][KT];
 #pragma unroll
         for (int t = 0; t < T; ++t)
             finish_acc<K, PREC>(acc[t], out[t]);
-        write_sums<K, PREC, T>(item, out, slot0, tstride, sub == 0);
+        Item next = item;
+        write_sums<K, PREC, T>(item, out, le >> ls, tstride, (le & (split - 1)) == 0, [&] {
+            it = __builtin_amdgcn_readfirstlane(take_item(a, cur, le, ticket));
+            if (it >= 0)
+                next = a.items[it];
+        });
+        if (it < 0)
+            return;
+        item = next;
     }
 }
 

@@ -84,14 +84,13 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
     constexpr int NA = AccCount<K, PREC>::value;
     const int lane = threadIdx.x;
     ItemCursor cur(a);
+    // uniform by construction; readfirstlane lets the compiler keep the item in SGPRs (and the
+    // scalar-broadcast variant's record reads as scalar loads)
+    int it = __builtin_amdgcn_readfirstlane(first_item(a, cur, lane));
+    if (it < 0)
+        return;
+    Item item = a.items[it];
     for (;;) {
-        // uniform by construction; readfirstlane lets the compiler keep the item in SGPRs (and the
-        // scalar-broadcast variant's record reads as scalar loads)
-        const int it = __builtin_amdgcn_readfirstlane(next_item(a, cur, lane));
-        if (it < 0)
-            break;
-
-        const Item item = a.items[it];
         const double lam = (PREC == 0) ? 1.0 : ldexp(1.0, item.level);
         const int ls = item.lsplit & (kItemWhole - 1);
         const int split = 1 << ls;
@@ -232,8 +231,10 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
             }
         }
 
+        int le = lane; // what follows from it is computed here, not held in registers over the pair loops
+        asm volatile("" : "+v"(le));
         if constexpr (PREC != 0)
-            redo_nonfinite_fp64<K>(a, item, acc, sub, split, tx, ty, tz, lam);
+            redo_nonfinite_fp64<K>(a, item, acc, le & (split - 1), split, tx, ty, tz, lam);
         for (int off = 1; off < split; off <<= 1) {
 #pragma unroll
             for (int t = 0; t < T; ++t)
@@ -241,11 +242,20 @@ __global__ void __launch_bounds__(kWave) p2p_items_sgpr_kernel(ItemArgs a, const
                 for (int k = 0; k < NA; ++k)
                     acc[t][k] += __shfl_xor(acc[t][k], off);
         }
+        const int ticket = request_item(a, cur, le);
         double out[T][KT];
 #pragma unroll
         for (int t = 0; t < T; ++t)
             finish_acc<K, PREC>(acc[t], out[t]);
-        write_sums<K, PREC, T>(item, out, slot0, tstride, sub == 0);
+        Item next = item;
+        write_sums<K, PREC, T>(item, out, le >> ls, tstride, (le & (split - 1)) == 0, [&] {
+            it = __builtin_amdgcn_readfirstlane(take_item(a, cur, le, ticket));
+            if (it >= 0)
+                next = a.items[it];
+        });
+        if (it < 0)
+            return;
+        item = next;
     }
 }
 
