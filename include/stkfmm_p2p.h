@@ -125,7 +125,7 @@ int stkfmm_p2p_eval(unsigned kernel, unsigned p2p, int precision, int nSrc, cons
 
 /* Device-resident variant: AoS device buffers, enqueued on `stream` (hipStream_t, 0 = null stream),
  * asynchronous.  No host memory is touched.  The device entries (this one, stkfmm_wall_eval_device,
- * stkfmm_p2p_vjp_device) keep per-device scratch (cached plans of each shape, workspaces) that
+ * stkfmm_p2p_vjp_device) keep per-device scratch (partial sums, cached plans of large shapes, workspaces) that
  * calls share: calls on one device must be ordered (one stream, or synchronised), or they race. */
 int stkfmm_p2p_eval_device(unsigned kernel, unsigned p2p, int precision, int nSrc, const double *d_srcCoord,
                            const double *d_srcValue, int nTrg, const double *d_trgCoord, double *d_trgValue,

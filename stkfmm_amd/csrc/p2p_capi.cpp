@@ -1195,8 +1195,8 @@ constexpr size_t kKernelCopyBytes = size_t(1) << 20;
 // d_tv) enqueues the device work on the null stream; with `stores` it overwrites d_tv (which may be host
 // memory), else it adds to it.
 // With engine copies each way and a cleared output 1,000 x 1,000 LapPGrad through evaluateKernel took 46 us,
-// so 33 (of them 16 us from the launches to the end of the synchronisation, 12 us of GPU time); 24 Ker_t
-// blocks 1.19 -> 0.94 ms.
+// so 33 (of them 16 us from the launches to the end of the synchronisation, 12 us of GPU time; 29 since the
+// Python entry's own part is shorter); 24 Ker_t blocks 1.19 -> 0.94 ms (0.87).
 template <class Eval>
 int host_roundtrip(size_t ks, size_t kt, int n_src, const double *sc, const double *sv, int n_trg,
                    const double *tc, double *tv, bool stores, Eval eval) {

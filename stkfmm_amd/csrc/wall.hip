@@ -4,7 +4,7 @@
 // User coordinates: the wall is the plane z = 0; the image of a source at (x, y, z) is (x, y, -z)
 // (the reference's setPoints, :40-80, shifts z to [0.5, 1) and places the image at 1 - z).
 // Bound by FP64 issue: 65,536 sources and targets, FP64, constituent sums (7 and 10 direct sums, ordered
-// points) -> source-and-image pairs: Stokes 24.3 -> 6.9 ms, RPY 49.9 -> 13.5 ms; 30,555 x 1,360 RPY 1.09 ->
+// points) -> source-and-image pairs: Stokes 24.3 -> 6.7 ms, RPY 49.9 -> 13.5 ms; 30,555 x 1,360 RPY 1.09 ->
 // 0.15 ms.  The Stokes pair's 42 FP64 operations, two reciprocal square roots (16 cycles each) and two masks
 // take about 6.2 ms at one operation per 4.2 cycles and SIMD.
 #include <hip/hip_runtime.h>
