@@ -523,7 +523,8 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     if (max_src <= 0 && persistent == 3) {
         max_src = 512; // per-group launches: split like a stand-alone direct sum of that group
     } else if (max_src <= 0) {
-        max_src = default_max_src(total_cost, concurrent);
+        max_src = precision == STKFMM_PREC_FP64 ? default_max_src_fp64(total_cost, concurrent, n_cu)
+                                                : default_max_src(total_cost, concurrent);
     }
     if (max_src < 1)
         max_src = 1;

@@ -215,6 +215,19 @@ inline long long default_max_src(long long total_cost, long long concurrent) {
     return m > 512 ? m : 512;
 }
 
+// FP64 plans of less work take smaller items: what the items cost beyond their pairs adds up to total_cost / m, the
+// tail is about m sources long and as much longer as more waves share a SIMD, which light kernels do, whose
+// items' own cost weighs more besides.  So m goes with the root of total_cost and of the resident waves; at least 192
+// sources.  512 -> 192 to 320, ms: PVel U-lists of 8,192 clustered points 0.077 -> 0.039, 32,768 0.165 -> 0.119,
+// 65,536 0.206 -> 0.157, 131,072 (lognormal) 0.272 -> 0.243; PVelGrad 0.135 -> 0.063, 0.252 -> 0.196, 0.329 -> 0.290,
+// 0.452 -> 0.442.  From 512 on the rule above.
+inline long long default_max_src_fp64(long long total_cost, long long concurrent, int n_cu) {
+    const double w = 16.0 * n_cu; // waves at four a SIMD
+    const double root = __builtin_sqrt((double)total_cost / w * ((double)concurrent / w));
+    const long long m = 64 * (long long)__builtin_ceil(13.0 * root / 64.0);
+    return m < 192 ? 192 : (m < 512 ? m : default_max_src(total_cost, concurrent));
+}
+
 // Workgroups per CU from which the default item size of a mixed-mode plan is counted.  Where a long source list
 // is cut decides which sources share an FP32 partial sum, and so the results' last FP32 bits: the cuts follow this
 // table (waves per SIMD of each micro-kernel, 0 to 24), not the register allocation of the build at hand.  In FP64

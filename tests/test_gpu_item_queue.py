@@ -48,3 +48,24 @@ def test_queues_give_the_same_bits(groups, uk, prec, bc):
         got = (out[0] - first)[host(perm)] / 2
         l2, mx = O.max_error(got, ref)
         assert l2 < FP64_TOL and mx < FP64_TOL, (l2, mx)
+
+
+# total work below and above each step of the default FP64 item size (192 .. 512 sources), against items of 512
+@pytest.mark.parametrize("groups,per", [(1, 191), (30, 193), (3000, 500), (9000, 900), (20000, 1300)])
+@pytest.mark.parametrize("uk", [2, 15])
+def test_default_fp64_items(uk, groups, per):
+    uk = S.UKER(uk)
+    say(f"default items uk={uk.name} groups={groups} sources={per}")
+    rng = np.random.default_rng(per)
+    ns, nt = 2000, groups * 2
+    sb = rng.integers(0, ns - per, groups)
+    src, trg, val = rng.random((ns, 3)), rng.random((nt, 3)), source_values(int(uk), ns, rng)
+    out = []
+    for tune in (None, dict(max_src_per_item=512)):
+        plan = S.Plan(uk, 0, ns, nt, np.arange(0, nt, 2), np.arange(0, nt, 2) + 2, None, np.arange(groups + 1), sb,
+                      sb + per, tune)
+        o = zeros(nt, S.uker_dims(uk)[1])
+        plan.execute(to_dev(src), to_dev(val), to_dev(trg), o)
+        out.append(host(o))
+    l2, mx = O.max_error(out[0], out[1])
+    assert l2 < FP64_TOL and mx < FP64_TOL, (l2, mx)
