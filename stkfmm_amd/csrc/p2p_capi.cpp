@@ -400,12 +400,22 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     // 3.58 ms, but draw more power, and the adjoint pass that follows in a training step then runs at a lower
     // clock (forward and adjoint in turn 12.17 ms as given, 12.04 ordered in LDS, 12.39 with the records).
     // (Mixed mode keeps the order it is given: its FP32 sums depend on it.)
-    if (untuned && single && precision == STKFMM_PREC_FP64 &&
+    const bool orders =
+        untuned && single && precision == STKFMM_PREC_FP64 &&
         direct_ordered_pays(precision, (long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]],
-                            (long long)grp_trg_end[0] - grp_trg_begin[0])) {
+                            (long long)grp_trg_end[0] - grp_trg_begin[0]);
+    if (orders) {
         tn.sort_points = 1;
         tn.targets_per_lane = 2;
     }
+    // the ordered copies are a choice of this entry: where there is no memory for them, the points as given
+    auto as_given = [&] {
+        (void)hipGetLastError();
+        stkfmm_tune t{};
+        t.targets_per_lane = 2;
+        return stkfmm_plan_create(plan_out, uk, precision, n_src, n_trg, n_groups, grp_trg_begin, grp_trg_end, grp_level,
+                                  grp_rng_ptr, rng_src_begin, rng_src_end, &t);
+    };
     // default targets per lane: 2, and 1 in mixed mode for the family members with many outputs or
     // much per-pair state, whose two-target loops run at lower occupancy: 262,144-point U-list, item
     // kernel + reduce (ms), T = 2 -> 1: PVelGrad 2.25 -> 2.03, LapQPGradGrad 2.34 -> 2.13,
@@ -731,7 +741,7 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         p->n_src_blks = n_src_blks;
         if ((r = upload(&p->d_sort_segs, segs, "sort segments")) || (r = upload(&p->d_sort_blks, blks, "sort blocks"))) {
             plan_free(p);
-            return r;
+            return orders ? as_given() : r;
         }
     }
     const size_t partial_elems = (size_t)p->n_items * p->KT * p->TT;
@@ -764,7 +774,7 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
         e = hipMalloc((void **)&p->d_recs, sizeof(double) * (size_t)p->n_copies * n_src * p->rec_words);
     if (e != hipSuccess) {
         plan_free(p);
-        return hip_error(e, "plan workspace");
+        return orders ? as_given() : hip_error(e, "plan workspace");
     }
     *plan_out = p;
     return STKFMM_OK;
