@@ -270,16 +270,28 @@ int stkfmm_plan_create(stkfmm_plan **plan, int uker, int precision, int n_src, i
  * NULL: identity).  src_value holds the first kdim values of each source; for
  * STKFMM_UKER_STOKES_PVEL_FUSED src_value holds the 4 single-layer values and src_value2 the 9
  * double-layer values of the same point (src_value2 is ignored for other micro-kernels).
+ * trg_value may overlap any input: every input is read before any output is written.  Where they may
+ * overlap the sums take a pass more; without a permutation the library sees the rows that are written,
+ * [0, n_trg), but perm (entries >= 0) may send them anywhere behind trg_value's first row.
+ * stkfmm_plan_execute_rows is told the number of rows of trg_value (perm's entries are below it).
  * Device arrays, enqueued on `stream`, asynchronous. */
 int stkfmm_plan_execute(stkfmm_plan *plan, const stkfmm_array *src_coord, const stkfmm_array *src_value,
                         const stkfmm_array *src_value2, const stkfmm_array *trg_coord,
                         const stkfmm_out_array *trg_value, const int *d_trg_perm, void *stream);
+int stkfmm_plan_execute_rows(stkfmm_plan *plan, const stkfmm_array *src_coord, const stkfmm_array *src_value,
+                             const stkfmm_array *src_value2, const stkfmm_array *trg_coord,
+                             const stkfmm_out_array *trg_value, const int *d_trg_perm, long long trg_rows,
+                             void *stream);
 
 /* Capture plan_execute with these exact arguments into a HIP graph held by the plan; subsequent
  * stkfmm_plan_launch_graph calls replay it.  Re-capturing replaces the previous graph. */
 int stkfmm_plan_capture_graph(stkfmm_plan *plan, const stkfmm_array *src_coord, const stkfmm_array *src_value,
                               const stkfmm_array *src_value2, const stkfmm_array *trg_coord,
                               const stkfmm_out_array *trg_value, const int *d_trg_perm, void *stream);
+int stkfmm_plan_capture_graph_rows(stkfmm_plan *plan, const stkfmm_array *src_coord,
+                                   const stkfmm_array *src_value, const stkfmm_array *src_value2,
+                                   const stkfmm_array *trg_coord, const stkfmm_out_array *trg_value,
+                                   const int *d_trg_perm, long long trg_rows, void *stream);
 int stkfmm_plan_launch_graph(stkfmm_plan *plan, void *stream);
 
 /* statistics: pairs = sum over groups of n_trg * n_src; n_items = work items; n_tiles = target tiles */

@@ -794,15 +794,17 @@ class Plan:
     def execute(self, src_coord, src_value, trg_coord, trg_value, src_value2=None, perm=None, stream=None):
         """trg_value(perm[i]) += ScaleFactor * sum over the work list (device tensors, any 2-D strides)."""
         (a, b, c, d, e), p = self._args(src_coord, src_value, trg_coord, trg_value, src_value2, perm)
-        _check(lib().stkfmm_plan_execute(self._h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c),
-                                         ctypes.byref(d), ctypes.byref(e), p, _stream_handle(stream)))
+        _check(lib().stkfmm_plan_execute_rows(self._h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c),
+                                              ctypes.byref(d), ctypes.byref(e), p, trg_value.shape[0],
+                                              _stream_handle(stream)))
         return trg_value
 
     def capture_graph(self, src_coord, src_value, trg_coord, trg_value, src_value2=None, perm=None, stream=None):
         """Capture execute(...) with these tensors into a HIP graph; replay with launch_graph()."""
         (a, b, c, d, e), p = self._args(src_coord, src_value, trg_coord, trg_value, src_value2, perm)
-        _check(lib().stkfmm_plan_capture_graph(self._h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c),
-                                               ctypes.byref(d), ctypes.byref(e), p, _stream_handle(stream)))
+        _check(lib().stkfmm_plan_capture_graph_rows(self._h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c),
+                                                    ctypes.byref(d), ctypes.byref(e), p, trg_value.shape[0],
+                                                    _stream_handle(stream)))
         self._keep = (src_coord, src_value, trg_coord, trg_value, src_value2, perm)
 
     def launch_graph(self, stream=None):

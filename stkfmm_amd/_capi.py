@@ -43,8 +43,8 @@ KER_T_UKER = {n: (i if i < 13 else i + 1) for i, n in enumerate(KER_T_NAMES)}
 EXPORTS = [
     "stkfmm_last_error", "stkfmm_get_kernel_dimension", "stkfmm_get_kernel_name", "stkfmm_get_uker",
     "stkfmm_uker_dims", "stkfmm_evaluate_kernel", "stkfmm_p2p_eval", "stkfmm_p2p_eval_device",
-    "stkfmm_ker_eval", "stkfmm_plan_create", "stkfmm_plan_execute", "stkfmm_plan_capture_graph",
-    "stkfmm_plan_launch_graph", "stkfmm_plan_stats", "stkfmm_plan_set_timing", "stkfmm_plan_kernel_ms",
+    "stkfmm_ker_eval", "stkfmm_plan_create", "stkfmm_plan_execute", "stkfmm_plan_execute_rows",
+    "stkfmm_plan_capture_graph", "stkfmm_plan_capture_graph_rows", "stkfmm_plan_launch_graph", "stkfmm_plan_stats", "stkfmm_plan_set_timing", "stkfmm_plan_kernel_ms",
     "stkfmm_plan_destroy", "stkfmm_tree_build", "stkfmm_tree_info", "stkfmm_tree_get", "stkfmm_tree_destroy",
     "stkfmm_p2p_vjp_device", "stkfmm_device_info", "stkfmm_tree_leaf_corners", "stkfmm_surface_count",
     "stkfmm_surface", "stkfmm_box_surfaces_device", "stkfmm_get_s2m_uker", "stkfmm_wall_evaluate",
@@ -79,6 +79,8 @@ def _declare(L):
     oarr = ctypes.POINTER(StkOutArray)
     L.stkfmm_plan_execute.argtypes = [c_void_p, arr, arr, arr, arr, oarr, c_void_p, c_void_p]
     L.stkfmm_plan_capture_graph.argtypes = [c_void_p, arr, arr, arr, arr, oarr, c_void_p, c_void_p]
+    L.stkfmm_plan_execute_rows.argtypes = [c_void_p, arr, arr, arr, arr, oarr, c_void_p, c_longlong, c_void_p]
+    L.stkfmm_plan_capture_graph_rows.argtypes = [c_void_p, arr, arr, arr, arr, oarr, c_void_p, c_longlong, c_void_p]
     L.stkfmm_plan_launch_graph.argtypes = [c_void_p, c_void_p]
     L.stkfmm_plan_stats.argtypes = [c_void_p, ctypes.POINTER(c_longlong), iptr, iptr, iptr]
     L.stkfmm_plan_set_timing.argtypes = [c_void_p, c_int]

@@ -219,7 +219,7 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
         a.scale = uker_scale(uk);
         a.n_src = nSrc;
         a.n_trg = nTrg;
-        a.two_phase = direct_out_overlaps(a, ks, ks1, kt);
+        a.two_phase = direct_out_overlaps(a, nTrg, ks, ks1, kt);
         const DirectLayout l = direct_layout_uk(uk, precision, direct_targets_per_lane(precision, kt, nTrg), nSrc, nTrg,
                                                 n_cu);
         if ((e = launch_direct(uk, precision, a, l, s)) != hipSuccess)

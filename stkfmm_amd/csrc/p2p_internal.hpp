@@ -2,6 +2,8 @@
 // (p2p_capi.cpp) of libstkfmm_p2p.so.  Not part of the public C ABI.
 #pragma once
 
+#include <cstdint>
+
 #include <hip/hip_runtime.h>
 
 namespace stkp2p {
@@ -317,9 +319,24 @@ int uker_run(int uk);
 // device memory for the chunks' partial sums of the direct-sum entries on the current device
 // (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
 int direct_partial_ptr(double **out, bool host);
-// out shares memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
-// the item and reduce kernels do
-bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt);
+// out may share memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
+// the item and reduce kernels do.  Without a permutation the rows written are [0, n_trg); through one they are
+// any of the output's out_rows, which the host does not see, and any from row 0 on where that is not known (-1).
+inline bool direct_out_overlaps(const DirectArgs &a, long long out_rows, int ks, int ks1, int kt) {
+    const long long rows = a.perm ? out_rows : a.n_trg;
+    if (rows == 0)
+        return false;
+    const auto last = [](const double *p, long long n, int k, long long s, long long fs) {
+        return (unsigned long long)(uintptr_t)p + sizeof(double) * ((n - 1) * s + (k - 1) * fs);
+    };
+    const unsigned long long o0 = (uintptr_t)a.out.p;
+    const unsigned long long o1 = rows < 0 ? ~0ull : last(a.out.p, rows, kt, a.out.s, a.out.fs);
+    const auto meets = [&](const DArr &x, long long n, int k) {
+        return k > 0 && o0 <= last(x.p, n, k, x.s, x.fs) && (uintptr_t)x.p <= o1;
+    };
+    return meets(a.sc, a.n_src, 3) || meets(a.v1, a.n_src, ks1) || meets(a.v2, a.n_src, ks - ks1) ||
+           meets(a.tc, a.n_trg, 3);
+}
 // dst[0, n) = src[0, n) by a kernel (small host-to-device copies)
 hipError_t launch_copy(const double *src, double *dst, size_t n, hipStream_t s);
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s);

@@ -209,16 +209,6 @@ void direct_args_layout(DirectArgs &a, const DirectLayout &l) {
     a.two_phase = a.two_phase || l.chunks > 1;
 }
 
-bool direct_out_overlaps(const DirectArgs &a, int ks, int ks1, int kt) {
-    const auto last = [](long long n, int k, long long s, long long fs) { return (n - 1) * s + (k - 1) * fs; };
-    const double *o0 = a.out.p, *o1 = o0 + last(a.n_trg, kt, a.out.s, a.out.fs);
-    const auto meets = [&](const DArr &x, long long n, int k) {
-        return k > 0 && x.p <= o1 && o0 <= x.p + last(n, k, x.s, x.fs);
-    };
-    return meets(a.sc, a.n_src, 3) || meets(a.v1, a.n_src, ks1) || meets(a.v2, a.n_src, ks - ks1) ||
-           meets(a.tc, a.n_trg, 3);
-}
-
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s) {
     if (!a.two_phase)
         return hipSuccess;

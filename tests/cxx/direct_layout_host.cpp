@@ -1,0 +1,27 @@
+// direct_layout_host.cpp -- test harness: the host rules of the direct sums (p2p_direct_layout.hpp,
+// p2p_internal.hpp) behind C functions, so tests/test_direct_layout.py can check them without a GPU.  Built by
+// stkfmm_amd/csrc/Makefile.  Not part of the library.
+#include "../../stkfmm_amd/csrc/p2p_direct_layout.hpp"
+
+using namespace stkp2p;
+
+// direct_out_overlaps of views given as (first byte address, row stride, component stride) in x[3]
+extern "C" int direct_overlaps_host(const unsigned long long *sc, const unsigned long long *v1,
+                                    const unsigned long long *v2, const unsigned long long *tc,
+                                    const unsigned long long *out, int perm, long long out_rows, int n_src,
+                                    int n_trg, int ks, int ks1, int kt) {
+    static const int some_perm = 0;
+    const auto in = [](const unsigned long long *x) {
+        return DArr{(const double *)(uintptr_t)x[0], (long long)x[1], (long long)x[2]};
+    };
+    DirectArgs a{};
+    a.sc = in(sc);
+    a.v1 = in(v1);
+    a.v2 = in(v2);
+    a.tc = in(tc);
+    a.out = OArr{(double *)(uintptr_t)out[0], (long long)out[1], (long long)out[2]};
+    a.perm = perm ? &some_perm : nullptr;
+    a.n_src = n_src;
+    a.n_trg = n_trg;
+    return direct_out_overlaps(a, out_rows, ks, ks1, kt);
+}

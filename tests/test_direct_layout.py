@@ -1,0 +1,75 @@
+"""The host rules of the direct sums (stkfmm_amd/csrc/p2p_direct_layout.hpp, p2p_internal.hpp), compiled for the CPU
+by tests/cxx/direct_layout_host.cpp."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from tests.conftest import ROOT
+
+LIB = os.path.join(ROOT, "tests", "cxx", "libdirect_layout_host.so")
+
+
+@pytest.fixture(scope="module")
+def lib():
+    if not os.path.exists(LIB):
+        pytest.skip("tests/cxx/libdirect_layout_host.so not built (make -C stkfmm_amd/csrc)")
+    return ctypes.CDLL(LIB)
+
+
+def view(first_double, stride, fstride=1):
+    return (ctypes.c_ulonglong * 3)(2 ** 20 + 8 * first_double, stride, fstride)
+
+
+def perm_rows(rows):
+    """The permutation's presence and the rows it may reach."""
+    return int(rows is not None), ctypes.c_longlong(-1 if rows is None else rows)
+
+
+# the output's first double and rows [0, n_trg) x 3 against four inputs of 3 columns; a field of 6,000 rows of 3
+# begins at double 0, other arrays lie at 100,000 and more
+FAR = 200_000
+OVERLAPS = [
+    # out, rows a permutation may reach (None: no permutation, -1: not known), source values, overlap
+    (0, None, FAR, False),
+    (0, None, 0, True),
+    (0, None, 2_999, True),          # the last value of row 999
+    (0, None, 3_000, False),         # row 1,000
+    (15_000, None, 12_000 - 1, False),
+    (15_000, None, 12_000, False),   # rows [4,000, 5,000) before rows [5,000, 6,000)
+    (15_000, None, 12_001, True),
+    (0, -1, 15_000, True),           # rows 5,000 and on, through a permutation to the same rows
+    (0, 6_000, 15_000, True),
+    (0, 5_001, 15_000, True),
+    (0, 5_000, 15_000, False),
+    (0, 6_000, 0, True),
+    (15_000, -1, 0, False),          # rows [0, 1,000): all in front of the output's first row
+    (15_000, -1, 12_001, True),
+    (0, 6_000, FAR, False),
+    (0, -1, FAR, True),
+    (FAR + 50_000, -1, FAR, False),
+]
+
+
+@pytest.mark.parametrize("out,rows,sv,expected", OVERLAPS)
+@pytest.mark.parametrize("which", range(4))
+def test_output_over_an_input_is_seen(lib, out, rows, sv, expected, which):
+    """Each input in turn (source coordinates, first and second source values, target coordinates) where the output
+    may be; the others in front of everything."""
+    n = 1000
+    arrays = [view(-100_000 + 4_000 * k, 3) for k in range(4)]
+    arrays[which] = view(sv, 3)
+    got = lib.direct_overlaps_host(*arrays, view(out, 3), *perm_rows(rows), n, n, 6, 3, 3)
+    assert bool(got) == expected
+
+
+def test_overlap_of_strided_views(lib):
+    """Columns of one tensor of seven: the extents meet, whatever lies between them."""
+    t = [view(100 * 7 * k + c, 7) for k, c in ((0, 0), (0, 3), (0, 6))]
+    far = view(FAR, 3)
+    assert lib.direct_overlaps_host(t[0], far, far, far, t[1], *perm_rows(None), 100, 100, 3, 3, 3)
+    assert not lib.direct_overlaps_host(far, far, far, view(700, 7), t[1], *perm_rows(None), 100, 100, 3, 3, 3)
+    # component-major: component 2 of 50 rows ends at double 149
+    assert lib.direct_overlaps_host(view(0, 1, 50), far, far, far, view(149, 3), *perm_rows(None), 50, 50, 3, 3, 3)
+    assert not lib.direct_overlaps_host(view(0, 1, 50), far, far, far, view(150, 3), *perm_rows(None), 50, 50, 3, 3, 3)
