@@ -30,7 +30,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // partial sums of the chunked direct sums of the other entries, which may run beside a no-alloc call: one array
 // for the device entries, whose calls the caller orders, and one for the host entries, which run under a lock
-static __device__ __align__(256) double direct_partial[2][16 * kDirectPartialTargets];
+static __device__ __align__(256) double direct_partial[2][kDirectPartial];
 
 // device addresses of the two arrays on each device (the host-side names are not device addresses)
 void *g_scratch_ptr[kMaxDevices] = {}, *g_partial_ptr[kMaxDevices] = {};
@@ -142,7 +142,7 @@ int direct_partial_ptr(double **out, bool host) {
         return report_error(STKFMM_ERR_HIP, "direct sum: hipGetDevice failed");
     void *p = nullptr;
     const int rc = symbol_ptr(dev, g_partial_ptr, HIP_SYMBOL(direct_partial), "direct_partial", &p);
-    *out = (double *)p + (host ? 16 * kDirectPartialTargets : 0);
+    *out = (double *)p + (host ? kDirectPartial : 0);
     return rc;
 }
 } // namespace stkp2p

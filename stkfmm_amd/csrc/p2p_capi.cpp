@@ -1178,7 +1178,7 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
                                          DArr{tc, 3, 1}, OArr{tv, kt, 1}, nullptr, n_trg, partial);
         a.store = store;
         // (an output over an input, with more targets than the fixed array holds, goes on to a plan)
-        if (!a.two_phase || (long long)l.chunks * n_trg * kt <= 16 * kDirectPartialTargets) {
+        if (!a.two_phase || (long long)l.chunks * n_trg * kt <= kDirectPartial) {
             HIP_TRY(launch_direct(uk, prec, a, l, s), "direct sum launch");
             return STKFMM_OK;
         }

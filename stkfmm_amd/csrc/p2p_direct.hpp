@@ -53,8 +53,15 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// waves per SIMD asked of the compiler: four where that takes a few registers off and no spills, so that two
+// workgroups of eight waves share a CU
+template <int UK, int PREC> struct DirectMinWaves {
+    static constexpr int value = (UK == 11 && PREC == 0) || (UK == 13 && PREC != 0) ? 4 : 1;
+};
+
 template <int UK, int PREC, int T>
-__global__ void __launch_bounds__(kWave *kDirectWaves) p2p_direct_kernel(DirectArgs a) {
+__global__ void __launch_bounds__(kWave *kDirectWaves)
+__attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct_kernel(DirectArgs a) {
     using K = typename UkerOf<UK>::type;
     using L = DirectLds<K, PREC>;
     constexpr int KL = L::KL, KLP = L::KLP, KT = K::KT, KS = K::KS, KS1 = K::KS1, TT = kWave * T;

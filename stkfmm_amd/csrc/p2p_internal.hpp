@@ -114,8 +114,8 @@ struct DirectArgs {
 };
 struct DirectLayout;
 void direct_args_layout(DirectArgs &a, const DirectLayout &l);
-// the chunks' partial sums hold at most this many targets' outputs (16 MiB at 16 outputs)
-constexpr long long kDirectPartialTargets = 131072;
+// the chunks' partial sums, in doubles, at most (16 MiB)
+constexpr long long kDirectPartial = 2097152;
 
 // XCD-contiguous work mapping.  Workgroups of a launch are dealt to MI355X's 8 XCDs round-robin
 // (workgroup b runs on XCD b % 8), each XCD with its own L2.  A launch of 8*ceil(n/8) workgroups that
@@ -317,7 +317,7 @@ hipError_t items_sgpr_occupancy(int uk, int prec, int T, int *blocks_per_cu);
 // direct sum: one launch, and a second one over the partial sums when there are several chunks
 int uker_run(int uk);
 // device memory for the chunks' partial sums of the direct-sum entries on the current device
-// (kDirectPartialTargets x 16 doubles, part of the library's image: never allocated, moved or freed)
+// (kDirectPartial doubles, part of the library's image: never allocated, moved or freed)
 int direct_partial_ptr(double **out, bool host);
 // out may share memory with an input (rows [0, n) of each view): the two-phase form reads everything first, as
 // the item and reduce kernels do.  Without a permutation the rows written are [0, n_trg); through one they are

@@ -17,7 +17,7 @@ namespace stkp2p {
 
 template <int UK, int T>
 static hipError_t launch_wall_t(DirectArgs &a, const DirectCost &cost, int n_cu, hipStream_t s) {
-    const DirectLayout l = direct_layout(0, T, cost, kSrcTile, a.n_src, a.n_trg, n_cu);
+    const DirectLayout l = direct_layout(0, T, cost, UkerOf<UK>::type::KT, kSrcTile, a.n_src, a.n_trg, n_cu);
     direct_args_layout(a, l);
     const hipError_t e = launch_direct_one<UK, 0, T>(a, l, s);
     return e != hipSuccess ? e : launch_direct_reduce(a, l.chunks, UkerOf<UK>::type::KT, s);

@@ -25,3 +25,12 @@ extern "C" int direct_overlaps_host(const unsigned long long *sc, const unsigned
     a.n_trg = n_trg;
     return direct_out_overlaps(a, out_rows, ks, ks1, kt);
 }
+
+// the cut of an n_src x n_trg sum of micro-kernel outputs kt (mixed mode: FP32 runs of `run` sources) on n_cu CUs, T
+// targets per lane: out = {units, chunks, chunk_tiles, waves, unit, ls, tail_begin, tail_ls}
+extern "C" void direct_layout_host(int prec, int T, int kt, int run, int n_src, int n_trg, int n_cu, int *out) {
+    const DirectLayout l = direct_layout(prec, T, direct_cost(prec, kt), kt, run, n_src, n_trg, n_cu);
+    const int v[8] = {l.units, l.chunks, l.chunk_tiles, l.waves, l.unit, l.ls, l.tail_begin, l.tail_ls};
+    for (int k = 0; k < 8; ++k)
+        out[k] = v[k];
+}

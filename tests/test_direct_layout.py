@@ -73,3 +73,42 @@ def test_overlap_of_strided_views(lib):
     # component-major: component 2 of 50 rows ends at double 149
     assert lib.direct_overlaps_host(view(0, 1, 50), far, far, far, view(149, 3), *perm_rows(None), 50, 50, 3, 3, 3)
     assert not lib.direct_overlaps_host(view(0, 1, 50), far, far, far, view(150, 3), *perm_rows(None), 50, 50, 3, 3, 3)
+
+
+PARTIAL = 2 ** 21  # doubles of the partial-sum array
+
+
+def layout(lib, prec, T, kt, n_src, n_trg, run=16, n_cu=256):
+    out = (ctypes.c_int * 8)()
+    lib.direct_layout_host(prec, T, kt, run, n_src, n_trg, n_cu, out)
+    return dict(zip(("units", "chunks", "chunk_tiles", "waves", "unit", "ls", "tail_begin", "tail_ls"), out))
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kt", [1, 3, 4, 6, 7, 10, 16])
+def test_cut_covers_the_sum(lib, prec, kt):
+    """Every target has a unit, every source tile a chunk, every chunk a tile; the chunks' sums fit their array."""
+    rng = np.random.default_rng(10 * kt + prec)
+    sizes = (10 ** rng.uniform(0, 6, (300, 2))).astype(int).tolist()
+    for n_src, n_trg in sizes + [[1, 1], [64, 128], [65, 129], [16_000, 100_000], [4_000, 1_000_000]]:
+        for T in (1, 2):
+            c = layout(lib, prec, T, kt, n_src, n_trg)
+            tiles = (n_src + 63) // 64
+            assert c["chunks"] == 1 or c["chunks"] * n_trg * kt <= PARTIAL
+            assert (c["chunks"] - 1) * c["chunk_tiles"] < tiles <= c["chunks"] * c["chunk_tiles"]
+            whole = c["units"] - (1 if c["tail_ls"] else 0)
+            assert (whole - 1) * c["unit"] < max(c["tail_begin"], 1) and whole * c["unit"] >= c["tail_begin"]
+            assert c["tail_begin"] == n_trg or (prec and n_trg - c["tail_begin"] < 64 * T and c["tail_ls"])
+            assert c["unit"] == 64 * T >> c["ls"] and 1 <= c["waves"] <= 8
+
+
+# bounded by 131,072 targets' worth of chunks whatever the outputs: 6.05, 6.1, 6.1 and 3.7 workgroups a CU, whose
+# last, partly filled round is as long as each of the others
+@pytest.mark.parametrize("n_src,n_trg", [(16_000, 33_000), (16_000, 50_000), (16_000, 100_000), (120_000, 120_000)])
+def test_targets_a_little_over_a_round(lib, n_src, n_trg):
+    """Light kernels' sums whose units would be a little more than whole rounds of workgroups come in so many chunks
+    that the last round is an eighth or less of the whole."""
+    for prec in (0, 1):
+        c = layout(lib, prec, 2, 4, n_src, n_trg)
+        rounds = c["units"] * c["chunks"] / 256
+        assert rounds >= 8, rounds
