@@ -53,15 +53,16 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// waves per SIMD asked of the compiler: four where that takes a few registers off and no spills, so that two
-// workgroups of eight waves share a CU
-template <int UK, int PREC> struct DirectMinWaves {
-    static constexpr int value = (UK == 11 && PREC == 0) || (UK == 13 && PREC != 0) ? 4 : 1;
-};
+// How the lanes of a workgroup hold its targets: a lane each, several lanes a target, or (FP64) either
+enum class Lanes { own, shared, any };
 
-template <int UK, int PREC, int T>
-__global__ void __launch_bounds__(kWave *kDirectWaves)
-__attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct_kernel(DirectArgs a) {
+// One workgroup's part of the sum.  In mixed mode each form of the source loop is a body of its own: side by side in
+// one, they keep a set of the FP64 accumulators in registers each (two targets per lane, LapPGradGrad 167 VGPRs,
+// apart 128; PVelLaplacian 150, 123; traction 152, 125; PVelGrad 240, 172: a wave less per SIMD than the item
+// kernels).  16,000 x 33,000: LapPGradGrad 516 -> 483 us, traction 543 -> 515, RegFTVelOmega 966 -> 861; 16,000 x
+// 260,000 PVelGrad 8.6 -> 7.2 ms; 8192^2 Stokeslet 50 -> 49 us.
+template <int UK, int PREC, int T, Lanes LANES>
+__device__ __forceinline__ void direct_unit(const DirectArgs &a, double *smem) {
     using K = typename UkerOf<UK>::type;
     using L = DirectLds<K, PREC>;
     constexpr int KL = L::KL, KLP = L::KLP, KT = K::KT, KS = K::KS, KS1 = K::KS1, TT = kWave * T;
@@ -70,7 +71,6 @@ __attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct
     // a run's first source on its own where the item kernels take it so: its products then start the
     // sums, which decides which of them is rounded (f/r + r b: one FMA of either product)
     constexpr bool PEEL = MixedPeel<K>::value && RUN == kMixedAccBlock;
-    extern __shared__ __align__(16) double smem[];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int W = (int)blockDim.x >> 6;
@@ -78,9 +78,11 @@ __attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct
     float *const rows = reinterpret_cast<float *>(sm + 3 * kSrcTile);
 
     // this workgroup's targets, and how its lanes share them
-    int ls = a.ls, tb = (int)blockIdx.x * a.unit, te = tb + min(a.unit, a.n_trg - tb);
+    int ls = LANES == Lanes::own ? 0 : a.ls, tb = (int)blockIdx.x * a.unit, te = tb + min(a.unit, a.n_trg - tb);
     bool runs = PREC != 0; // lanes share a target by whole FP32 runs
-    if (PREC != 0 && a.tail_ls > 0) {
+    if (LANES == Lanes::own) {
+        te = min(te, a.tail_begin);
+    } else if (PREC != 0 && a.tail_ls > 0) {
         if ((int)blockIdx.x == (int)gridDim.x - 1) {
             ls = a.tail_ls;
             tb = a.tail_begin;
@@ -210,7 +212,7 @@ __attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct
                     pair64(j);
             }
         } else {
-            if (ls == 0) {
+            if constexpr (LANES == Lanes::own) {
                 for (int g = 0; g < n; g += RUN) {
                     const int e = min(g + RUN, n);
                     clear_runs();
@@ -332,6 +334,24 @@ __attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct
             }
         }
     }
+}
+
+// waves per SIMD asked of the compiler: four where that takes a few registers off and no spills, so that two
+// workgroups of eight waves share a CU
+template <int UK, int PREC> struct DirectMinWaves {
+    static constexpr int value = (UK == 11 && PREC == 0) ? 4 : 1;
+};
+
+template <int UK, int PREC, int T>
+__global__ void __launch_bounds__(kWave *kDirectWaves)
+__attribute__((amdgpu_waves_per_eu(DirectMinWaves<UK, PREC>::value))) p2p_direct_kernel(DirectArgs a) {
+    extern __shared__ __align__(16) double smem[];
+    if constexpr (PREC == 0)
+        direct_unit<UK, PREC, T, Lanes::any>(a, smem);
+    else if (a.ls == 0 && (a.tail_ls == 0 || blockIdx.x + 1 < gridDim.x))
+        direct_unit<UK, PREC, T, Lanes::own>(a, smem);
+    else
+        direct_unit<UK, PREC, T, Lanes::shared>(a, smem);
 }
 
 template <int UK, int PREC, int T>

@@ -89,9 +89,9 @@ inline DirectLayout direct_layout(int prec, int T, const DirectCost &cost, int k
 // the layout of micro-kernel uk's direct sum, T targets per lane
 inline DirectLayout direct_layout_uk(int uk, int prec, int T, int n_src, int n_trg, int n_cu) {
     DirectCost cost = direct_cost(prec, uker_kt(uk));
-    // regularised force and torque with the rotation, and the fused PVel in FP64: as more than six outputs (137-160
-    // VGPRs; 16,000 x 50,000 of the first 1.97 -> 1.62 ms FP64, 1.74 -> 1.37 mixed, with the chunks above)
-    if (T == 2 && (uk == 20 || (uk == 13 && prec == 0)))
+    // regularised force and torque with the rotation, and the fused PVel: as more than six outputs (152 and 160
+    // VGPRs; 16,000 x 50,000 of the first 1.97 -> 1.62 ms, with the chunks above)
+    if (prec == 0 && (uk == 20 || uk == 13))
         cost.max_waves = kDirectWaves / 2;
     return direct_layout(prec, T, cost, uker_kt(uk), uker_run(uk), n_src, n_trg, n_cu);
 }
