@@ -136,9 +136,9 @@ int stkfmm_p2p_eval_device(unsigned kernel, unsigned p2p, int precision, int nSr
  * arguments, semantics and kernels; it calls no hipMalloc/hipFree.  Its work list and partial sums
  * live in a fixed 64 MiB device array per GPU, held from the library's load until the process ends,
  * so a sum whose targets alone need more (about 2M targets at 4 output values, 512K at 16) returns
- * STKFMM_ERR_ARG.  Below 16,384 sources or targets (in FP64 also below 2^29 pairs), and while the
- * plan-based entry's partial sums fit the array, the results are bitwise identical to it; otherwise the same pairs are summed in another
- * grouping (the plan-based entry orders larger sums' points along a Morton curve; this one keeps the
+ * STKFMM_ERR_ARG.  Below 16,384 sources or targets (in FP64 also below 2^29 pairs) and 2^32 pairs, and
+ * while the plan-based entry's partial sums fit the array, the results are bitwise identical to it; otherwise
+ * the same pairs are summed in another grouping (the plan-based entry orders larger sums' points along a Morton curve; this one keeps the
  * caller's order, and cuts the sources into fewer chunks when its array is the limit).
  * Every call on one GPU uses that GPU's array: calls that overlap on one device (different streams,
  * or several host threads without ordering) race and corrupt each other's results. */

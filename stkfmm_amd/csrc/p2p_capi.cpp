@@ -366,9 +366,21 @@ static bool direct_sorts_points(int prec, int n_src, int n_trg) {
     return direct_ordered_pays(prec, n_src, n_trg) || !direct_sizes(n_src, n_trg);
 }
 
-// direct sums that are one launch
-static bool direct_in_one_call(int uk, int prec, int n_src, int n_trg) {
+// direct sums that one launch can do, and those that it does
+static bool direct_can_launch(int uk, int prec, int n_src, int n_trg) {
     return !direct_sorts_points(prec, n_src, n_trg) && direct_in_one_launch(prec, uk);
+}
+static bool direct_in_one_call(int uk, int prec, int n_src, int n_trg) {
+    return direct_can_launch(uk, prec, n_src, n_trg) && !direct_items_pay(n_src, n_trg);
+}
+// s is being captured (a plan cannot be made then)
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
 }
 
 extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision, int n_src, int n_trg,
@@ -703,7 +715,9 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
 
     // A single untuned direct sum below the sizes that pay for ordered points: one launch instead of queue
     // reset, item kernel and reduce.  The item list above stays for stkfmm_plan_stats.
-    if (untuned && single && p->n_items > 0 && direct_in_one_call(uk, precision, n_src, n_trg)) {
+    if (untuned && single && p->n_items > 0 && direct_can_launch(uk, precision, n_src, n_trg) &&
+        !direct_items_pay((long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]],
+                          (long long)grp_trg_end[0] - grp_trg_begin[0])) {
         const int r0 = grp_rng_ptr[0];
         p->direct = true;
         p->dt_begin = grp_trg_begin[0];
@@ -1105,12 +1119,14 @@ int direct_plan(int uk, int prec, int n_src, int n_trg, stkfmm_plan **out) {
     // One target group.  From kDirectSortMin sources and targets its points are ordered along a Morton
     // curve at every call: T = 2, and in FP64 the scalar-broadcast records (65,536^2 PVel FP64 4.05 ->
     // 3.76 ms, 131,072^2 14.72 -> 14.24 ms against LDS staging of the ordered points).  Below that, where
-    // one launch does not serve (direct_in_one_launch): one target per lane under 32,768 targets.
+    // one launch does not serve (direct_in_one_call): one target per lane under 32,768 targets, and the records in
+    // FP64 from there.
     stkfmm_tune tn{};
     const bool sort = n_trg >= kDirectSortMin && n_src >= kDirectSortMin;
     tn.sort_points = sort ? 1 : 0;
-    tn.targets_per_lane = sort || n_trg >= 32768 ? 2 : 1;
-    tn.broadcast = (sort && prec == STKFMM_PREC_FP64) ? 1 : 0;
+    const bool two = sort || n_trg >= 32768;
+    tn.targets_per_lane = two ? 2 : 1;
+    tn.broadcast = (two && prec == STKFMM_PREC_FP64) ? 1 : 0;
     stkfmm_plan *p = nullptr;
     int rc = stkfmm_plan_create(&p, uk, prec, n_src, n_trg, 1, &gb, &ge, nullptr, gp, &rb, &re, &tn);
     if (rc)
@@ -1168,7 +1184,12 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
         return set_error(STKFMM_ERR_ARG, "NULL buffer");
     const int ks = uker_ks(uk), ks1 = uker_ks1(uk), kt = uker_kt(uk);
     int rc;
-    if (direct_in_one_call(uk, prec, n_src, n_trg)) {
+    // (a sum that the items do faster takes the launch all the same where their plan cannot be made)
+    const bool can_launch = direct_can_launch(uk, prec, n_src, n_trg), items = direct_items_pay(n_src, n_trg);
+    stkfmm_plan *p = nullptr;
+    if (can_launch && items && !capturing(s) && (rc = direct_plan(uk, prec, n_src, n_trg, &p)))
+        (void)hipGetLastError();
+    if (can_launch && !p) {
         int n_cu = 0;
         double *partial = nullptr;
         if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial, store)))
@@ -1183,8 +1204,7 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
             return STKFMM_OK;
         }
     }
-    stkfmm_plan *p = nullptr;
-    if ((rc = direct_plan(uk, prec, n_src, n_trg, &p)))
+    if (!p && (rc = direct_plan(uk, prec, n_src, n_trg, &p)))
         return rc;
     stkfmm_array a_sc{sc, 3, 1}, a_sv{sv, ks, 1}, a_sv2{sv + ks1, ks, 1}, a_tc{tc, 3, 1};
     stkfmm_out_array a_tv{tv, kt, 1};

@@ -270,6 +270,16 @@ inline bool direct_ordered_pays(int prec, long long n_src, long long n_trg) {
     return n_src >= kDirectSortMin && n_trg >= kDirectSortMin && (prec != 0 || n_src * n_trg >= 1LL << 29);
 }
 
+// Direct sums that leave the one launch for the item kernels, whose waves take work as they become free: from 2^32
+// pairs and 8,192 sources on (so with 262,144 targets and more: from 16,384 sources the points are ordered) the launch
+// has no chunks left to even out its last round (kDirectPartial).  16,000 x 500,000, one launch and items, ms: FP64
+// LapPGrad 5.25 and 4.95, PVel 7.39 and 6.75, RPY 9.50 and 8.46; mixed Stokeslet 4.67 and 4.35, PVelGrad 14.5 and 12.6.
+// With fewer sources the launch is even or ahead (1,500 x 3,000,000 mixed RPY 3.34 and 3.61), and below 2^32 pairs the
+// plan that the items need, 1 to 2 ms at a shape's first call, costs too much.
+constexpr bool direct_items_pay(long long n_src, long long n_trg) {
+    return n_src >= 8192 && n_trg > n_src && n_src * n_trg >= 1LL << 32;
+}
+
 // lanes per target of a tile of n targets (log2): the largest power of two, at most 16, that still
 // fits the tile's 64*T lanes
 __host__ __device__ inline int tile_lsplit(int n, int TT) {

@@ -34,3 +34,5 @@ extern "C" void direct_layout_host(int prec, int T, int kt, int run, int n_src, 
     for (int k = 0; k < 8; ++k)
         out[k] = v[k];
 }
+
+extern "C" int direct_items_pay_host(long long n_src, long long n_trg) { return direct_items_pay(n_src, n_trg); }

@@ -112,3 +112,12 @@ def test_targets_a_little_over_a_round(lib, n_src, n_trg):
         c = layout(lib, prec, 2, 4, n_src, n_trg)
         rounds = c["units"] * c["chunks"] / 256
         assert rounds >= 8, rounds
+
+
+@pytest.mark.parametrize("n_src,n_trg,items", [(16_000, 500_000, True), (16_000, 268_435, False), (16_000, 268_436, True),
+                                               (8_192, 524_287, False), (8_192, 524_288, True), (8_191, 600_000, False),
+                                               (500_000, 16_000, False), (1_500, 3_000_000, False),
+                                               (2 ** 30, 2 ** 30 - 1, False)])
+def test_sums_that_go_to_the_items(lib, n_src, n_trg, items):
+    got = lib.direct_items_pay_host(ctypes.c_longlong(n_src), ctypes.c_longlong(n_trg))
+    assert bool(got) == items
