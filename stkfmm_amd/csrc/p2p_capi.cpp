@@ -1173,7 +1173,8 @@ int ws_get(int slot, size_t n, double **out) {
     return STKFMM_OK;
 }
 
-// the device-pointer entries' sum; store (only where direct_in_one_call): tv = sum instead of tv += sum
+// the device-pointer entries' sum; store (the host-pointer entries', on the null stream): tv = sum instead of tv +=
+// sum, with a partial-sum array of their own
 int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *sv, int n_trg, const double *tc,
                    double *tv, hipStream_t s, bool store = false) {
     if (n_src < 0 || n_trg < 0)
@@ -1206,6 +1207,8 @@ int eval_device_uk(int uk, int prec, int n_src, const double *sc, const double *
     }
     if (!p && (rc = direct_plan(uk, prec, n_src, n_trg, &p)))
         return rc;
+    if (store) // a plan adds
+        HIP_TRY(hipMemsetAsync(tv, 0, sizeof(double) * kt * n_trg, s), "clear output");
     stkfmm_array a_sc{sc, 3, 1}, a_sv{sv, ks, 1}, a_sv2{sv + ks1, ks, 1}, a_tc{tc, 3, 1};
     stkfmm_out_array a_tv{tv, kt, 1};
     return plan_enqueue(p, &a_sc, &a_sv, &a_sv2, &a_tc, &a_tv, nullptr, n_trg, s, false);
@@ -1238,8 +1241,8 @@ constexpr size_t kKernelCopyBytes = size_t(1) << 20;
 // A host-pointer evaluation: the three inputs are packed into the pinned buffer and moved to the device; the
 // result comes back through the pinned buffer, after one synchronisation; the caller's trgValue += result
 // is then done here (the same additions as on the device, since 0 + x is exact).  eval(d_sc, d_sv, d_tc,
-// d_tv) enqueues the device work on the null stream; with `stores` it overwrites d_tv (which may be host
-// memory), else it adds to it.
+// d_tv) enqueues the device work on the null stream and overwrites d_tv; where its kernels write each value once
+// (`stores`), d_tv may be host memory.
 // With engine copies each way and a cleared output 1,000 x 1,000 LapPGrad through evaluateKernel took 46 us,
 // so 33 (of them 16 us from the launches to the end of the synchronisation, 12 us of GPU time; 29 since the
 // Python entry's own part is shorter); 24 Ker_t blocks 1.19 -> 0.94 ms (0.87).
@@ -1262,8 +1265,6 @@ int host_roundtrip(size_t ks, size_t kt, int n_src, const double *sc, const doub
         HIP_TRY(launch_copy(h, d, n_in, nullptr), "copy inputs");
     else
         HIP_TRY(hipMemcpyAsync(d, h, sizeof(double) * n_in, hipMemcpyHostToDevice, nullptr), "copy inputs");
-    if (!stores)
-        HIP_TRY(hipMemsetAsync(d_tv, 0, sizeof(double) * n_tv, nullptr), "clear output");
     rc = eval(d, d + n_sc, d + n_sc + n_sv, d_tv);
     if (rc) {
         (void)hipStreamSynchronize(nullptr);
@@ -1288,7 +1289,7 @@ int eval_host_uk(int uk, int prec, int n_src, const double *sc, const double *sv
     const bool stores = direct_in_one_call(uk, prec, n_src, n_trg);
     return host_roundtrip(uker_ks(uk), uker_kt(uk), n_src, sc, sv, n_trg, tc, tv, stores,
                           [&](const double *d_sc, const double *d_sv, const double *d_tc, double *d_tv) {
-                              return eval_device_uk(uk, prec, n_src, d_sc, d_sv, n_trg, d_tc, d_tv, nullptr, stores);
+                              return eval_device_uk(uk, prec, n_src, d_sc, d_sv, n_trg, d_tc, d_tv, nullptr, true);
                           });
 }
 
