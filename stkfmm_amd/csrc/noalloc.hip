@@ -208,7 +208,7 @@ extern "C" int stkfmm_p2p_eval_device_noalloc(unsigned kernel, unsigned p2p, int
     // for the mixed-mode sums that do not run so (direct_in_one_launch), and for those above the array's
     // size: their longer chunks need not start on a whole source tile, which decides the sources each
     // FP32 partial sum holds.
-    if ((precision == STKFMM_PREC_FP64 || (!limited && direct_in_one_launch(precision, uk))) && nSrc <= (1 << 30) && nTrg <= (1 << 30)) {
+    if ((precision == STKFMM_PREC_FP64 || (!limited && direct_in_one_launch(precision, uk))) && direct_sizes(nSrc, nTrg)) {
         DirectArgs a{};
         a.sc = DArr{d_srcCoord, 3, 1};
         a.v1 = DArr{d_srcValue, ks, 1};

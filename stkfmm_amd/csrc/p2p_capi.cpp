@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstdarg>
@@ -359,8 +360,6 @@ static void group_tiles(int n, int TT, bool pieces, std::vector<int> &counts) {
     }
 }
 
-// sizes a direct sum's 32-bit indices cover
-static bool direct_sizes(int n_src, int n_trg) { return n_src <= (1 << 30) && n_trg <= (1 << 30); }
 // direct sums whose entry orders the points (or whose sizes one launch does not cover)
 static bool direct_sorts_points(int prec, int n_src, int n_trg) {
     return direct_ordered_pays(prec, n_src, n_trg) || !direct_sizes(n_src, n_trg);
@@ -1336,6 +1335,8 @@ int wall_device(unsigned kernel, const double *sc, const double *sv, int n, cons
                 hipStream_t s, bool store = false) {
     int n_cu = 0, rc;
     double *partial = nullptr;
+    if (n > INT_MAX - kSrcTile) // (the kernel counts whole tiles)
+        return set_error(STKFMM_ERR_ARG, "wall images: %d sources exceed the index range", n);
     if ((rc = device_cu_count(&n_cu)) || (rc = direct_partial_ptr(&partial, store)))
         return rc;
     const int ks = kernel == STKFMM_KERNEL_Stokes ? 3 : 4, kt = kernel == STKFMM_KERNEL_Stokes ? 3 : 6;
@@ -1362,7 +1363,7 @@ int wall_device(unsigned kernel, const double *sc, const double *sv, int n, cons
         a.v1.p = a.v2.p = w + 3 * N;
         a.tc.p = w + (3 + ks) * N;
     }
-    // target slabs keep the launch inside its index range
+    // target slabs keep the launches inside their index range (direct_sizes)
     const int slab = 1 << 29;
     const double *t_first = a.tc.p;
     for (long long t0 = 0; t0 < m; t0 += slab) {

@@ -6,6 +6,7 @@
 namespace stkp2p {
 
 constexpr int kDirectWaves = 8; // waves per workgroup, at most
+constexpr long long kMaxGridThreads = 1LL << 32; // of a launch, along each axis: below this
 
 struct DirectLayout {
     int T;           // targets per lane
@@ -69,6 +70,10 @@ inline DirectLayout direct_layout(int prec, int T, const DirectCost &cost, int k
             l.waves = cost.max_waves;
             while (l.waves > 1 && l.waves / 2 >= l.chunk_tiles)
                 l.waves /= 2;
+            while (l.waves > 1 && (long long)l.units * kWave * l.waves >= kMaxGridThreads)
+                l.waves /= 2;
+            if ((long long)l.units * kWave * l.waves >= kMaxGridThreads)
+                continue;
             const double rounds = (double)((l.chunk_tiles + l.waves - 1) / l.waves);
             const double wave_t = rounds * (kStage + (kWave >> ls) * T * cost.pair);
             const long long wgs = ((long long)l.units * l.chunks + n_cu - 1) / n_cu;

@@ -113,6 +113,10 @@ struct DirectArgs {
     int ls, unit, tail_begin, tail_ls, chunk_tiles; // DirectLayout
 };
 struct DirectLayout;
+// workgroups of 256 threads that add up the chunks of n_trg targets, 64 each
+inline unsigned direct_reduce_blocks(int n_trg) { return ((unsigned)n_trg + 63u) / 64u; }
+// sizes that a direct sum's 32-bit indices, and launches of fewer than 2^32 threads, cover
+constexpr bool direct_sizes(int n_src, int n_trg) { return n_src <= 1 << 30 && n_trg <= (1 << 30) - 64; }
 void direct_args_layout(DirectArgs &a, const DirectLayout &l);
 // the chunks' partial sums, in doubles, at most (16 MiB)
 constexpr long long kDirectPartial = 2097152;

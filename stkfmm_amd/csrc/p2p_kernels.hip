@@ -212,7 +212,7 @@ void direct_args_layout(DirectArgs &a, const DirectLayout &l) {
 hipError_t launch_direct_reduce(const DirectArgs &a, int chunks, int kt, hipStream_t s) {
     if (!a.two_phase)
         return hipSuccess;
-    hipLaunchKernelGGL(direct_reduce_kernel, dim3((unsigned)((a.n_trg + 63) / 64)), dim3(256), 0, s, a, chunks, kt);
+    hipLaunchKernelGGL(direct_reduce_kernel, dim3(direct_reduce_blocks(a.n_trg)), dim3(256), 0, s, a, chunks, kt);
     return hipGetLastError();
 }
 

@@ -36,3 +36,15 @@ extern "C" void direct_layout_host(int prec, int T, int kt, int run, int n_src, 
 }
 
 extern "C" int direct_items_pay_host(long long n_src, long long n_trg) { return direct_items_pay(n_src, n_trg); }
+
+// threads of the launches over the targets: the sum's along x, the reduction's
+extern "C" void direct_threads_host(int prec, int T, int kt, int max_waves, int n_src, int n_trg, long long *out) {
+    DirectCost cost = direct_cost(prec, kt);
+    if (max_waves > 0)
+        cost.max_waves = max_waves;
+    const DirectLayout l = direct_layout(prec, T, cost, kt, 16, n_src, n_trg, 256);
+    out[0] = (long long)l.units * kWave * l.waves;
+    out[1] = direct_reduce_blocks(n_trg) * 256LL;
+}
+
+extern "C" int direct_sizes_host(int n_src, int n_trg) { return direct_sizes(n_src, n_trg); }

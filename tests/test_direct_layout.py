@@ -121,3 +121,15 @@ def test_targets_a_little_over_a_round(lib, n_src, n_trg):
 def test_sums_that_go_to_the_items(lib, n_src, n_trg, items):
     got = lib.direct_items_pay_host(ctypes.c_longlong(n_src), ctypes.c_longlong(n_trg))
     assert bool(got) == items
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("T,kt,waves", [(1, 10, 0), (1, 16, 0), (2, 3, 0), (2, 6, 0), (1, 6, 8), (2, 3, 8)])
+@pytest.mark.parametrize("n_trg", [2 ** 29, 2 ** 30 - 129, 2 ** 30 - 128, 2 ** 30 - 127, 2 ** 30 - 64])
+def test_launches_stay_below_2_32_threads(lib, prec, T, kt, waves, n_trg):
+    """The largest sums, and (eight waves a workgroup) the wall images' slabs of 2^29 targets."""
+    out = (ctypes.c_longlong * 2)()
+    assert lib.direct_sizes_host(2 ** 30, n_trg) and not lib.direct_sizes_host(1, 2 ** 30 - 63)
+    for n_src in (1, 64, 300, 1_000, 20_000, 10 ** 6):
+        lib.direct_threads_host(prec, T, kt, waves, n_src, n_trg, out)
+        assert 0 < out[0] < 2 ** 32 and 0 < out[1] < 2 ** 32, (n_src, out[0], out[1])
