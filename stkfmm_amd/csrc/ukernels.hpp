@@ -177,7 +177,8 @@ __host__ __device__ constexpr double post_for(int k) {
 
 // FP64 pair form with accumulators of its own: micro-kernels that declare ACC64 accumulate ACC64 sums per
 // target with eval64<M>(a, dx, dy, dz, f) (M = false: pairs known to have r2 > 0) and turn them into the
-// outputs (before post()) once per target and work item with finish64(a, out).  It lets terms common to
+// outputs (before post()) once per target and work item with finish64(a, out).  Powers of w = 2/r up to w^5 hold
+// for separations of 1e-61 to 1e61, as the reference's own do at best.  It lets terms common to
 // several outputs be summed once: symmetric and antisymmetric halves of a tensor, the multiple of the
 // unit matrix in its diagonal, constant factors.  eval<double> is then one pair through both.
 template <class K, class = void> struct HasEval64 { static constexpr bool value = false; };

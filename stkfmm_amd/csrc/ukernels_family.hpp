@@ -13,7 +13,10 @@
 // Coincident pairs: s = 0 gives n = 0 and every output carries at least one factor of s, so they
 // contribute exactly 0, as the reference's masked approx_rsqrt does.
 //
-// FP64 has the range for powers of w = 2/r (twice_rsqrt) up to w^7, which saves the three products of n,
+// FP64 takes powers of w = 2/r (twice_rsqrt) up to w^7, which every output stands for separations of 9e-44 to 4e43
+// (LapQPGradGrad; the others, up to w^5, from 1e-61 to 1e61): farther than the reference's own powers reach in each
+// kernel (1e-34 to 1e34 with r^-9, 1e-43 to 1e44 with r^-7, 1e-61 to 1e62 with r^-5), though not as far as the
+// unit-direction form (1e-61, 1e-76 or 1e-102).  It saves the three products of n,
 // and accumulates in a basis of its own (ACC64, ukernels.hpp): a symmetric tensor as six sums, an
 // antisymmetric part as three, the multiple of the unit matrix once, constant factors at the end.  The
 // kernels are bound by FP64 issue, so a pair's time follows its operations; 262,144-point U-list, 1.06e9
