@@ -411,10 +411,12 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     // 3.58 ms, but draw more power, and the adjoint pass that follows in a training step then runs at a lower
     // clock (forward and adjoint in turn 12.17 ms as given, 12.04 ordered in LDS, 12.39 with the records).
     // (Mixed mode keeps the order it is given: its FP32 sums depend on it.)
-    const bool orders =
-        untuned && single && precision == STKFMM_PREC_FP64 &&
-        direct_ordered_pays(precision, (long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]],
-                            (long long)grp_trg_end[0] - grp_trg_begin[0]);
+    // The copies are as long as the arrays, so that the ranges have to be most of them.
+    const long long rng_src = single ? (long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]] : 0;
+    const long long rng_trg = single ? (long long)grp_trg_end[0] - grp_trg_begin[0] : 0;
+    const bool orders = untuned && single && precision == STKFMM_PREC_FP64 &&
+                        direct_ordered_pays(precision, rng_src, rng_trg) && 2 * rng_src >= n_src &&
+                        2 * rng_trg >= n_trg;
     if (orders) {
         tn.sort_points = 1;
         tn.targets_per_lane = 2;
@@ -715,8 +717,7 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
     // A single untuned direct sum below the sizes that pay for ordered points: one launch instead of queue
     // reset, item kernel and reduce.  The item list above stays for stkfmm_plan_stats.
     if (untuned && single && p->n_items > 0 && direct_can_launch(uk, precision, n_src, n_trg) &&
-        !direct_items_pay((long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]],
-                          (long long)grp_trg_end[0] - grp_trg_begin[0])) {
+        !direct_items_pay(rng_src, rng_trg)) {
         const int r0 = grp_rng_ptr[0];
         p->direct = true;
         p->dt_begin = grp_trg_begin[0];
