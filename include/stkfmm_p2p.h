@@ -135,7 +135,8 @@ int stkfmm_p2p_eval_device(unsigned kernel, unsigned p2p, int precision, int nSr
 /* No counterpart in the reference: stkfmm_p2p_eval_device for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, semantics and kernels; it calls no hipMalloc/hipFree.  Its work list and partial sums
- * live in a fixed 64 MiB device array per GPU, held from the library's load until the process ends,
+ * live in a fixed 64 MiB device array per GPU, held from the library's load until the process ends (as are
+ * two of 16 MiB for the partial sums of the device and of the host entries),
  * so a sum whose targets alone need more (about 2M targets at 4 output values, 512K at 16) returns
  * STKFMM_ERR_ARG.  Below 16,384 sources or targets (in FP64 also below 2^29 pairs) and 2^32 pairs, and
  * while the plan-based entry's partial sums fit the array, the results are bitwise identical to it; otherwise

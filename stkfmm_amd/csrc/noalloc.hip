@@ -1,16 +1,16 @@
 // noalloc.hip -- stkfmm_p2p_eval_device_noalloc: the device direct sum with no device allocation.
 //
-// The work list of a single-group direct sum is regular (target tiles of 64*T consecutive targets,
-// each against the sources in chunks of max_src), so a small kernel writes it on the device instead
-// of the host uploading it, and everything the item and reduce kernels need beyond the caller's
-// inputs and output -- items, source ranges, tiles, the queue bounds and counter, the per-item
-// partial sums -- lives in one file-scope device array, `scratch`, of kScratchBytes per device.
-// The kernels are the ones the cached-plan entry (stkfmm_p2p_eval_device) runs on points in the
-// caller's order: below 16,384 sources or targets (where that entry does not order the points along a
-// Morton curve) and while the partial sums fit, the tiling and chunking are the plan's as well and the
-// two entries give bitwise identical results; otherwise the same pairs are summed in another grouping
-// (no point ordering here, which would need copies of the points; above the plan's partial-sum size,
-// fewer and longer source chunks).
+// Everything a sum needs beyond the caller's inputs and output lives in one file-scope device array, `scratch`, of
+// kScratchBytes per device.  FP64, and mixed mode where the item list's partial sums would fit the array, is one
+// launch (p2p_direct.hpp) whose chunks' partial sums it holds.  The other mixed-mode sums (direct_in_one_launch, and
+// the larger ones) run the item kernels: the work list of a single-group direct sum is regular (target tiles of 64*T
+// consecutive targets, each against the sources in chunks of max_src), so a small kernel writes it on the device
+// instead of the host uploading it, and the array holds items, source ranges, tiles, the queue bounds and
+// counter, and the per-item partial sums.
+// Below 16,384 sources or targets (FP64: also below 2^29 pairs) and 2^32 pairs the entry that may allocate
+// (stkfmm_p2p_eval_device) sums in the same kernels and cuts, while its partial sums fit the array, and the two give
+// bitwise identical results; otherwise the same pairs are summed in another grouping (no point ordering here,
+// which would need copies of the points; above the plan's partial-sum size, fewer and longer source chunks).
 #include <hip/hip_runtime.h>
 
 #include <cstdio>

@@ -408,8 +408,8 @@ extern "C" int stkfmm_plan_create(stkfmm_plan **plan_out, int uk, int precision,
                         (long long)grp_rng_ptr[1] - grp_rng_ptr[0] == 1 && rng_src_begin && rng_src_end;
     // A large untuned FP64 one orders its points: PVel 65,536^2 3.90 -> 3.65 ms, PVelGrad 8.06 -> 7.82, Laplace
     // potential 1.97 -> 1.82.  Staged in LDS: the scalar-broadcast records of the device entries (direct_plan) take
-    // 3.58 ms, but draw more power, and the adjoint pass that follows in a training step then runs at a lower
-    // clock (forward and adjoint in turn 12.17 ms as given, 12.04 ordered in LDS, 12.39 with the records).
+    // 3.58 ms, but the adjoint pass that follows in a training step then runs at a lower clock (its cycles are the
+    // same, at 1.94 GHz for 2.00: forward and adjoint in turn 12.17 ms as given, 12.04 in LDS, 12.39 with the records).
     // (Mixed mode keeps the order it is given: its FP32 sums depend on it.)
     // The copies are as long as the arrays, so that the ranges have to be most of them.
     const long long rng_src = single ? (long long)rng_src_end[grp_rng_ptr[0]] - rng_src_begin[grp_rng_ptr[0]] : 0;

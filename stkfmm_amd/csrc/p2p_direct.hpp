@@ -1,4 +1,4 @@
-// p2p_direct.hpp -- one target group against one source range (a direct sum) in one launch.
+// p2p_direct.hpp -- one target group against one source range (a direct sum) in one launch, or one and a reduction.
 //
 // The item kernels give a 64*T-target tile and 512 or more sources to one wave, and a second launch
 // sums the waves' partial results.  A small sum then has a handful of waves on 256 CUs (1,000 x
@@ -7,11 +7,12 @@
 // w + W, ... from LDS of its own (no barrier inside the loop; the next tile's loads are in flight
 // while one is evaluated), the waves' sums meet in LDS at the end, and the caller's output is written
 // by the same launch.  A unit is 64*T >> ls targets: 2^ls lanes share a target and split each tile's
-// sources between them, which gives a sum of few targets enough workgroups.  Only when that is not
-// enough (fewer than ~100 targets against many sources) the sources are cut into chunks as well
-// (blockIdx.y), whose partial results [chunk][KT][n_trg] direct_reduce_kernel adds up.  The layout
-// comes from direct_layout (p2p_direct_layout.hpp).  Measured on MI355X, whole calls on resident points,
-// item kernel + reduce -> one launch: LapPGrad FP64 8192^2 95 -> 52 us (705 -> 1290 Gpair/s; bound by its
+// sources between them, which gives a sum of few targets enough workgroups.  Where CUs would idle all the
+// same, or the last round of workgroups be nearly empty, the sources are cut into chunks as well (blockIdx.y), whose
+// partial results [chunk][KT][n_trg] direct_reduce_kernel adds up in a second launch: 8192^2 in 8 chunks, 3,001 x
+// 2,503 in 6, 1,000^2 in one.  The layout is the cheapest by the cost model of direct_layout
+// (p2p_direct_layout.hpp).  Measured on MI355X, whole calls on resident points,
+// item kernel + reduce -> this kernel (+ reduction): LapPGrad FP64 8192^2 95 -> 52 us (705 -> 1290 Gpair/s; bound by its
 // FP64 issue from there, 45 us), Stokeslet mixed 3,001 x 2,503 82 -> 16 us of GPU time; 24 Ker_t blocks of
 // different sizes on host arrays 3.7 -> 1.2 ms (no work list to build and upload for a new size).
 //
