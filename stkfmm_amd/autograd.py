@@ -19,8 +19,9 @@ _ADJOINT_UKERS = frozenset(int(u) for u in (
 class P2PFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, uker, precision, src_coord, src_value, trg_coord):
+        uker = int(uker)
         if uker not in _ADJOINT_UKERS:
-            raise ValueError(f"no adjoint kernel for {UKER(int(uker)).name}")
+            raise ValueError(f"no adjoint kernel for {UKER(uker).name}")
         _, kt = uker_dims(uker)
         sc, sv, tc = src_coord.contiguous(), src_value.contiguous(), trg_coord.contiguous()
         out = torch.zeros((tc.shape[0], kt), dtype=torch.float64, device=tc.device)
