@@ -787,7 +787,7 @@ class Plan:
         else:
             _dev2d(trg_value, self.n_trg, self.kt, "trg_value")
         sv = _sarr(src_value)
-        sv2 = _sarr(src_value2) if src_value2 is not None else sv
+        sv2 = _sarr(src_value2) if self._fused else sv
         args = (_sarr(src_coord), sv, sv2, _sarr(trg_coord), _oarr(trg_value))
         return args, (None if perm is None else perm.data_ptr())
 
